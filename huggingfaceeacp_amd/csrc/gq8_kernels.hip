@@ -359,10 +359,9 @@ __global__ __launch_bounds__(kThreads) void kv_store_kernel(const float *__restr
 // Lane l of a wave owns the 32-element blocks l, l + 64, ... of an output row
 // (32 weight bytes = two 16-byte loads, one fp16 scale), dots them against
 // the same blocks of up to B activation rows staged in LDS with sdot4, and
-// accumulates scale * dot in double.  Each wave owns U consecutive output
-// rows; a workgroup (four waves) loops over the activation rows in groups of
-// B, so a multi-row step reads every weight row from HBM once.
-template <int B, int U>
+// accumulates scale * dot in double.  A wave owns an output row; a workgroup
+// (four waves) loops over the activation rows in groups of B.
+template <int B>
 __global__ __launch_bounds__(kThreads) void q8_product_kernel(
     const uint8_t *__restrict__ x8, int64_t x_elements, int x_row0, int rows,
     const uint8_t *__restrict__ w8, int inner, int outputs, float *__restrict__ y, int y_stride,
@@ -378,7 +377,7 @@ __global__ __launch_bounds__(kThreads) void q8_product_kernel(
     const int64_t wElements = (int64_t) outputs * inner;
     const uint16_t *wScales = reinterpret_cast<const uint16_t *>(w8 + wElements);
     const uint16_t *xScales = reinterpret_cast<const uint16_t *>(x8 + x_elements);
-    const int out0 = (blockIdx.x * (kThreads / 64) + wave) * U;
+    const int o = blockIdx.x * (kThreads / 64) + wave;
 
     for (int g = 0; g < rows; g += B) {
         const int gb = min(B, rows - g);
@@ -395,30 +394,20 @@ __global__ __launch_bounds__(kThreads) void q8_product_kernel(
         }
         __syncthreads();
 
-        double acc[U][B];
+        double acc[B];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int b = 0; b < B; ++b)
-                acc[u][b] = 0.0;
+        for (int b = 0; b < B; ++b)
+            acc[b] = 0.0;
 
         for (int blk = lane; blk < nb; blk += 64) {
-            int4 wa[U], wb[U];
-            double ws[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int o = out0 + u;
-                if (o < outputs) {
-                    const int4 *p = reinterpret_cast<const int4 *>(w8 + (int64_t) o * inner
-                                                                   + (int64_t) blk * kBlock);
-                    wa[u] = p[0];
-                    wb[u] = p[1];
-                    ws[u] = (double) half_value(wScales[(int64_t) o * nb + blk]);
-                } else {
-                    wa[u] = make_int4(0, 0, 0, 0);
-                    wb[u] = make_int4(0, 0, 0, 0);
-                    ws[u] = 0.0;
-                }
+            int4 wa = make_int4(0, 0, 0, 0), wb = make_int4(0, 0, 0, 0);
+            double ws = 0.0;
+            if (o < outputs) {
+                const int4 *p = reinterpret_cast<const int4 *>(w8 + (int64_t) o * inner
+                                                               + (int64_t) blk * kBlock);
+                wa = p[0];
+                wb = p[1];
+                ws = (double) half_value(wScales[(int64_t) o * nb + blk]);
             }
 #pragma unroll
             for (int b = 0; b < B; ++b) {
@@ -426,34 +415,27 @@ __global__ __launch_bounds__(kThreads) void q8_product_kernel(
                     const int4 *ap = reinterpret_cast<const int4 *>(sQ + b * inner + blk * kBlock);
                     const int4 a0 = ap[0], a1 = ap[1];
                     const double sa = sScale[b * nb + blk];
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        int d = 0;
-                        d = __builtin_amdgcn_sdot4(wa[u].x, a0.x, d, false);
-                        d = __builtin_amdgcn_sdot4(wa[u].y, a0.y, d, false);
-                        d = __builtin_amdgcn_sdot4(wa[u].z, a0.z, d, false);
-                        d = __builtin_amdgcn_sdot4(wa[u].w, a0.w, d, false);
-                        d = __builtin_amdgcn_sdot4(wb[u].x, a1.x, d, false);
-                        d = __builtin_amdgcn_sdot4(wb[u].y, a1.y, d, false);
-                        d = __builtin_amdgcn_sdot4(wb[u].z, a1.z, d, false);
-                        d = __builtin_amdgcn_sdot4(wb[u].w, a1.w, d, false);
-                        acc[u][b] += (double) d * (ws[u] * sa); // all three exact but the sum
-                    }
+                    int d = 0;
+                    d = __builtin_amdgcn_sdot4(wa.x, a0.x, d, false);
+                    d = __builtin_amdgcn_sdot4(wa.y, a0.y, d, false);
+                    d = __builtin_amdgcn_sdot4(wa.z, a0.z, d, false);
+                    d = __builtin_amdgcn_sdot4(wa.w, a0.w, d, false);
+                    d = __builtin_amdgcn_sdot4(wb.x, a1.x, d, false);
+                    d = __builtin_amdgcn_sdot4(wb.y, a1.y, d, false);
+                    d = __builtin_amdgcn_sdot4(wb.z, a1.z, d, false);
+                    d = __builtin_amdgcn_sdot4(wb.w, a1.w, d, false);
+                    acc[b] += (double) d * (ws * sa); // all three exact but the sum
                 }
             }
         }
 
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-#pragma unroll
-            for (int b = 0; b < B; ++b) {
-                const double total = wave_sum(acc[u][b]);
-                const int o = out0 + u;
-                if (lane == 0 && b < gb && o < outputs) {
-                    float *dst = y + (int64_t) (g + b) * y_stride + o;
-                    const double old = residual ? (double) *dst : 0.0;
-                    *dst = (float) (total + old);
-                }
+        for (int b = 0; b < B; ++b) {
+            const double total = wave_sum(acc[b]);
+            if (lane == 0 && b < gb && o < outputs) {
+                float *dst = y + (int64_t) (g + b) * y_stride + o;
+                const double old = residual ? (double) *dst : 0.0;
+                *dst = (float) (total + old);
             }
         }
     }
@@ -1007,14 +989,14 @@ hipError_t launch_kv_store(const float *k, const float *v, int src_stride, int r
 }
 
 namespace {
-template <int B, int U>
+template <int B>
 hipError_t product_with(const uint8_t *x8, int64_t xElements, int xRow0, int rows,
                         const uint8_t *w8, int inner, int outputs, float *y, int yStride,
                         int residual, hipStream_t stream)
 {
     const size_t lds = (size_t) B * inner + (size_t) B * (inner / kBlock) * sizeof(double);
-    const unsigned grid = blocks_for(outputs, (kThreads / 64) * U);
-    hipLaunchKernelGGL((q8_product_kernel<B, U>), dim3(grid), dim3(kThreads), lds, stream, x8,
+    const unsigned grid = blocks_for(outputs, kThreads / 64);
+    hipLaunchKernelGGL(q8_product_kernel<B>, dim3(grid), dim3(kThreads), lds, stream, x8,
                        xElements, xRow0, rows, w8, inner, outputs, y, yStride, residual);
     return hipGetLastError();
 }
@@ -1072,31 +1054,29 @@ hipError_t launch_q8_product(const uint8_t *x8, int x_rows_total, int x_row0, in
     const int64_t xElements = (int64_t) x_rows_total * inner;
     if (rows == 1)
         return launch_matvec(x8, xElements, x_row0, w8, inner, outputs, y, residual, stream);
-    if (q8_gemm_supported(rows, inner, outputs))
-        return launch_q8_gemm(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride,
-                              residual, stream);
-    int b = 8;
-    while (b > 1 && (b > rows || product_lds(b, inner) > kProductLdsLimit))
-        b >>= 1;
-    // rows per wave: 8 for a vocabulary-wide product, 4 for the feed-forward
-    // width, 1 where the matrix is too small to fill the chip otherwise
-    const int perWave = inner > 4096 ? 1 : (outputs >= 131072 ? 8 : (outputs >= 16384 ? 4 : 1));
-#define GQ8_PRODUCT(BB)                                                                      \
-    switch (perWave) {                                                                       \
-    case 8: return product_with<BB, 8>(x8, xElements, x_row0, rows, w8, inner, outputs, y,   \
-                                       y_stride, residual, stream);                          \
-    case 4: return product_with<BB, 4>(x8, xElements, x_row0, rows, w8, inner, outputs, y,   \
-                                       y_stride, residual, stream);                          \
-    default: return product_with<BB, 1>(x8, xElements, x_row0, rows, w8, inner, outputs, y,  \
-                                        y_stride, residual, stream);                         \
+    // a few rows of a narrow product: whole weight rows a wave stream better
+    // than the MFMA tiles do (2 rows of 16384 -> 2048: 13.4 against 19.3 us,
+    // of 2048 -> 2048: 4.0 against 4.6; even at 4 rows, 21.2 and 4.2 against
+    // 19.4 and 4.6; at 5 the tiles lead, 27 and 5.5 against 19.5 and 4.6).  A
+    // wide one (2 rows of 2048 -> 32768: 17.3 against 15.0) is the tiles'.
+    if (rows <= 4 && outputs < 16384) {
+        int b = 4;
+        while (b > 1 && (b > rows || product_lds(b, inner) > kProductLdsLimit))
+            b >>= 1;
+        switch (b) {
+        case 4:
+            return product_with<4>(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride,
+                                   residual, stream);
+        case 2:
+            return product_with<2>(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride,
+                                   residual, stream);
+        default:
+            return product_with<1>(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride,
+                                   residual, stream);
+        }
     }
-    switch (b) {
-    case 8: GQ8_PRODUCT(8);
-    case 4: GQ8_PRODUCT(4);
-    case 2: GQ8_PRODUCT(2);
-    default: GQ8_PRODUCT(1);
-    }
-#undef GQ8_PRODUCT
+    return launch_q8_gemm(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride, residual,
+                          stream);
 }
 
 size_t mqa_workspace_bytes(int rows, int heads, int head_dim, int max_keys)

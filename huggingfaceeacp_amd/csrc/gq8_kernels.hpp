@@ -47,10 +47,9 @@ hipError_t launch_kv_store(const float *k, const float *v, int src_stride, int r
                            const int *pos_ptr, int pos_value, hipStream_t stream);
 
 // x8: Q8 row buffer of x_rows_total rows; rows [x_row0, x_row0 + rows) are used.
-// Steps of kGemmMinRows rows or more whose inner size is a whole number of
-// 256-byte chunks run on the int8 MFMA GEMM (gq8_gemm.hip).
-constexpr int kGemmMinRows = 32;
-bool q8_gemm_supported(int rows, int inner, int outputs);
+// Several rows run on the int8 MFMA GEMM (gq8_gemm.hip), whose tile is chosen
+// by the product's shape, or for a few rows of a narrow product in
+// q8_product_kernel; one row in q8_matvec_kernel.
 // The gate|up product of a fused [2 F, inner] weight with GeGLU and its Q8
 // folded into the GEMM's epilogue: q8_out receives the [rows, F] Q8 row
 // buffer of the activations, debug_out (optional) their fp32 values.

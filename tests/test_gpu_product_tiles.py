@@ -1,0 +1,86 @@
+"""The multi-row product's tiles at their edges: every tile the choice can
+take, with rows and outputs that leave its last tiles partial, block counts
+that leave its last chunk partial or shorter than a chunk, a row stride past
+the outputs, and the residual."""
+import numpy as np
+import pytest
+
+import oracle as O
+from gpu_helpers import spread, to_device
+from huggingfaceeacp_amd import gemma_q8 as G
+
+pytestmark = pytest.mark.gpu
+
+# (rows, outputs): the tile the choice takes for them
+TILES = {
+    "whole rows a wave": (4, 70),
+    "16 x 16": (17, 34),
+    "16 x 16, two rounds": (33, 2050),
+    "32 x 16": (60, 2040),
+    "16 x 32": (35, 8210),
+    "32 x 64": (31, 9002),
+    "64 x 32": (130, 2046),
+    "64 x 64": (257, 2090),
+    "128 x 64": (2040, 2046),
+}
+
+
+@pytest.mark.parametrize("inner", [32, 96, 256, 1056, 1280])
+@pytest.mark.parametrize("tile", list(TILES))
+def test_product_tile_edges(torch_cuda, tile, inner):
+    torch = torch_cuda
+    rows, outputs = TILES[tile]
+    if inner > 256 and rows * outputs > 1 << 20:
+        inner = 768  # the oracle's time; still whole and several chunks
+    nb, stride = inner // 32, outputs + 3
+    w = O.quantize_int8_blocks(spread(inner * outputs, 91, 0.05))
+    q, s = O.quantize_row(spread(rows * inner, 92, 1.0))
+    x8 = np.concatenate([q.view(np.uint8), s.view(np.uint8)])
+    base = spread(rows * stride, 93, 1.0)
+    xd, wd = to_device(torch, x8), to_device(torch, w)
+    for residual in (False, True):
+        y = to_device(torch, base)
+        G.q8_product(xd.data_ptr(), wd.data_ptr(), rows, inner, outputs, y.data_ptr(), stride,
+                     residual=residual)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy().reshape(rows, stride)
+        before = base.reshape(rows, stride)
+        assert np.array_equal(got[:, outputs:], before[:, outputs:])
+        for r in sorted({0, 1, rows // 2, rows - 2, rows - 1} | set(range(0, rows, 37))):
+            ref = O.q8_matvec(q[r * inner:(r + 1) * inner], s[r * nb:(r + 1) * nb], w, outputs,
+                              inner).astype(np.float64)
+            if residual:
+                # the oracle's product is already fp32: half an ulp of it, then
+                # the stored sum's own half ulp
+                ref = ref + before[r, :outputs]
+                bound = 2.0 ** -24 * (np.abs(ref - before[r, :outputs]) + np.abs(ref)) + 1e-12
+            else:
+                # both round doubles that differ by sums in another order, a
+                # few 2^-53: the same fp32 or its neighbour
+                bound = 2.0 ** -23 * np.abs(ref) + 1e-12
+            assert np.all(np.abs(got[r, :outputs] - ref) <= bound), f"row {r}"
+
+
+@pytest.mark.parametrize("rows", [2, 16, 17, 33, 100])
+def test_prompt_rows_equal_single_steps(torch_cuda, rows):
+    """A prompt step's gate | up product with GeGLU folded in takes a tile by
+    its rows (16, 32, 64 or 128); each row's logits are those of one-row steps
+    through the separate product and GeGLU kernels."""
+    torch = torch_cuda
+    shape = G.DecoderShape(256, 2, 1, 128, 1, 16384, 512, 128, 128)
+    d = G.Decoder(shape)
+    for i in range(shape.tensor_count()):
+        sigma = 0.1 if i == 0 or shape.tensor_is_norm(i) else 0.06
+        d.load_tensor(i, O.normal_fill(0x7100 + i, sigma, shape.tensor_elements(i)))
+    ids = to_device(torch, O.prompt_ids(0xC0FFEE, shape.vocab, rows).astype(np.int32))
+    block = torch.empty(rows, shape.vocab, device="cuda")
+    d.begin_sequence()
+    d.step(ids.data_ptr(), rows, block.data_ptr(), rows)
+    single = torch.empty(1, shape.vocab, device="cuda")
+    d.set_fused(False)
+    d.begin_sequence()
+    for r in range(rows):
+        d.step(ids.data_ptr() + 4 * r, 1, single.data_ptr(), 1)
+        torch.cuda.synchronize()
+        # the same doubles in another order, rounded to fp32 at each store
+        assert torch.allclose(block[r], single[0], rtol=1e-5, atol=1e-6), f"row {r}"

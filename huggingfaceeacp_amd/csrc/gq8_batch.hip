@@ -759,7 +759,7 @@ __device__ inline void row_lane_fmac(double (&p)[K], double s, const double (&x)
 
 // C channels a lane (head width 64 C), H heads, G of them a workgroup
 // (blockIdx.z picks the group; the groups of one key tile share the tile's
-// rows through the L2), a split of per_split keys in tiles of kRowsTileKeys.
+// rows through the L2), a split of plan.per_split keys in tiles of kRowsTileKeys.
 // Scores: wave w takes a quarter of the channels and its lane l keys
 // t0 + l % 16 + 16 j (j < kLaneKeys) over the quarter's slice l / 16 of
 // 4 C channels, every head of the group; lane c of each 16-lane row holds
@@ -793,7 +793,7 @@ __global__ __launch_bounds__(kRowsThreads, 2) void attention_rows_kernel(RowsAtt
 
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int seq = blockIdx.y, split = blockIdx.x, hBase = blockIdx.z * G;
-    const int k0 = split * a.per_split;
+    const int k0 = split * a.plan.per_split;
     // the position first: its wait then counts only the loads before it
     const int pos = a.positions[seq];
     asm volatile("" ::: "memory");
@@ -858,7 +858,7 @@ __global__ __launch_bounds__(kRowsThreads, 2) void attention_rows_kernel(RowsAtt
     const int keyCount = pos + 1;
     if (k0 >= keyCount)
         return;
-    const int k1 = min(k0 + a.per_split, keyCount);
+    const int k1 = split + 1 < (int) gridDim.x ? min(k0 + a.plan.per_split, keyCount) : keyCount;
     const bool holdsNew = k1 == keyCount; // this split ends at the new position
 
     // RoPE (rope_kv_kernel's arithmetic) of the group's query heads and, in
@@ -1082,7 +1082,8 @@ __global__ __launch_bounds__(64) void attention_merge_rows_kernel(RowsAttentionA
     const int hd = a.head_dim, H = a.heads, qW = H * hd;
     const int quarters = hd / 64; // waves a head
     const int head = blockIdx.x / quarters, seq = blockIdx.y, t = threadIdx.x;
-    const int splits = (a.positions[seq] + a.per_split) / a.per_split; // keys: position + 1
+    const int splits = min((a.positions[seq] + a.plan.per_split) / a.plan.per_split, // keys: position + 1
+                           a.plan.splits);
     const int64_t first = (int64_t) seq * kRowsMaxSplits;
     const int o = head * hd + (blockIdx.x % quarters) * 64 + t;
     double part[kRowsMaxSplits];
@@ -1373,10 +1374,28 @@ bool rows_attention_supported(int heads, int kv_heads, int head_dim, int max_pos
            && max_positions <= kRowsMaxSplits * kRowsTileKeys * 64;
 }
 
-int rows_attention_split_keys(int max_positions)
+// One 80-key tile a split while 32 splits cover the keys (ranges of 4, 8, 16
+// and 32 splits, so a short row's step launches no more workgroups than it
+// uses), whole tiles a split beyond.  The line follows the keys of the step
+// and not the window: a split sized for an 8192-position window holds 320
+// keys, four tiles one after another, and 16 rows of 1088 keys then keep 128
+// workgroups busy for 35.1 us where 14 one-tile splits a row take 12.1.
+RowsAttentionPlan rows_attention_plan(int keys, int max_positions)
 {
-    const int span = kRowsMaxSplits * kRowsTileKeys;
-    return kRowsTileKeys * ((max_positions + span - 1) / span);
+    constexpr int kSpan = kRowsMaxSplits * kRowsTileKeys;
+    RowsAttentionPlan p{kRowsTileKeys, 4, 4 * kRowsTileKeys};
+    while (p.last_keys < keys && p.splits < kRowsMaxSplits) {
+        p.splits *= 2;
+        p.last_keys *= 2;
+    }
+    if (p.last_keys < keys) {
+        const int tiles = (keys + kSpan - 1) / kSpan;
+        p.per_split = tiles * kRowsTileKeys;
+        p.last_keys = tiles * kSpan;
+    }
+    p.last_keys = p.last_keys < max_positions ? p.last_keys : max_positions;
+    p.splits = (p.last_keys + p.per_split - 1) / p.per_split;
+    return p;
 }
 
 size_t rows_attention_workspace_doubles(int rows, int heads, int head_dim)
@@ -1384,15 +1403,15 @@ size_t rows_attention_workspace_doubles(int rows, int heads, int head_dim)
     return (size_t) rows * kRowsMaxSplits * heads * (head_dim + 2);
 }
 
-hipError_t launch_rows_attention(const RowsAttentionArgs &a, int rows, int max_positions,
-                                 hipStream_t stream)
+hipError_t launch_rows_attention(const RowsAttentionArgs &a, int rows, hipStream_t stream)
 {
     if (rows <= 0 || rows > kBatchRows || a.q8_rows < rows || !a.row_angles
-        || !rows_attention_supported(a.heads, 1, a.head_dim, max_positions)
-        || a.per_split != rows_attention_split_keys(max_positions) || a.max_positions != max_positions)
+        || !rows_attention_supported(a.heads, 1, a.head_dim, a.max_positions)
+        || a.plan.per_split <= 0 || a.plan.per_split % kRowsTileKeys != 0 || a.plan.splits <= 0
+        || a.plan.splits > kRowsMaxSplits)
         return hipErrorInvalidValue;
     const int groups = a.heads > kRowsHeadGroup ? a.heads / kRowsHeadGroup : 1;
-    const dim3 grid((max_positions + a.per_split - 1) / a.per_split, rows, groups);
+    const dim3 grid(a.plan.splits, rows, groups);
     const int C = a.head_dim / 64;
 #define GQ8_ROWS_ATTENTION(CC, HH)                                                              \
     hipLaunchKernelGGL((attention_rows_kernel<CC, HH, (HH > kRowsHeadGroup ? kRowsHeadGroup : HH)>), grid, \

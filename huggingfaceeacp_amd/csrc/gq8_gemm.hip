@@ -451,7 +451,7 @@ constexpr int kMaxTileRows = 65535; // the grid's y extent
 const TileCost kProductTiles[] = {
     {128, 64, 20.2, 18.2, launch_tile<Tile128x64, false, false>},
     {64, 64, 11.3, 10.0, launch_tile<Tile64x64, false, true>},
-    {64, 32, 6.6, 6.0, launch_tile<Tile64x32, false, true>},
+    {64, 32, 6.6, 5.6, launch_tile<Tile64x32, false, true>},
     {32, 64, 6.8, 6.4, launch_tile<Tile32x64, false, true>},
     {16, 32, 3.6, 2.3, launch_tile<Tile16x32, false, true>},
     {32, 16, 2.7, 2.7, launch_tile<Tile32x16, false, true>},

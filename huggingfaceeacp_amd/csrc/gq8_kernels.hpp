@@ -155,10 +155,17 @@ hipError_t launch_tile_weights(const uint8_t *w8, int inner, int outputs, uint8_
 // q | k | v; the keys [0, positions[r]] of sequence r's caches (the layer's
 // base for sequence 0, cache_stride elements a sequence) are attended after
 // the new key and value are appended at positions[r].  The merged row goes to
-// row r of a Q8 row buffer of q8_rows rows.  per_split is
-// rows_attention_split_keys(max_positions); ws_o / ws_ml hold
-// rows_attention_workspace_doubles.
+// row r of a Q8 row buffer of q8_rows rows.  plan is rows_attention_plan of
+// the longest row's keys; ws_o / ws_ml hold rows_attention_workspace_doubles.
 constexpr int kRowsMaxSplits = 32;
+// The split of a step whose longest row attends `keys` keys: `splits`
+// workgroups a row and head group of per_split keys each, for steps of up to
+// last_keys keys (a captured step replays over that range; the last split
+// takes whatever lies past it).
+struct RowsAttentionPlan {
+    int per_split, splits, last_keys;
+};
+RowsAttentionPlan rows_attention_plan(int keys, int max_positions);
 struct RowsAttentionArgs {
     const float *qkv;
     int qkv_stride;
@@ -169,16 +176,14 @@ struct RowsAttentionArgs {
     int max_positions;        // rows of each cache (the bound of speculative reads)
     int heads, head_dim;
     float scale;
-    int per_split;
+    RowsAttentionPlan plan;
     double *ws_o, *ws_ml;
     uint8_t *q8;
     int q8_rows;
 };
 bool rows_attention_supported(int heads, int kv_heads, int head_dim, int max_positions);
-int rows_attention_split_keys(int max_positions);
 size_t rows_attention_workspace_doubles(int rows, int heads, int head_dim);
-hipError_t launch_rows_attention(const RowsAttentionArgs &a, int rows, int max_positions,
-                                 hipStream_t stream);
+hipError_t launch_rows_attention(const RowsAttentionArgs &a, int rows, hipStream_t stream);
 
 // The gate | up product with GeGLU fused: w8 is the stacked [gate; up]
 // tensor (2 intermediate rows), and GeGLU of row m's products goes, as Q8, to

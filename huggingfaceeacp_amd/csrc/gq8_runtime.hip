@@ -18,6 +18,7 @@
 #include <cstring>
 #include <random>
 #include <string>
+#include <map>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -2149,7 +2150,7 @@ struct gq8_batch {
     bool tiled = false;
     void *argmaxWorkspace = nullptr;
     size_t argmaxWorkspaceBytes = 0;
-    hipGraphExec_t graph = nullptr;
+    std::map<int, hipGraphExec_t> graphs; // the captured step of each key-count range, by its last key
     std::vector<void *> allocations;
 };
 
@@ -2242,9 +2243,17 @@ int refresh_tiled(gq8_batch *b)
             return status_;                  \
     } while (0)
 
+// The attention split of the batch's step `ahead` steps from its host
+// positions.
+gq8::RowsAttentionPlan batch_plan(const gq8_batch *b, int ahead)
+{
+    const int longest = *std::max_element(b->hostPositions.begin(), b->hostPositions.end());
+    return gq8::rows_attention_plan(longest + ahead + 1, b->d->shape.max_positions);
+}
+
 // One lockstep step: every sequence's token at its position, its argmax into
 // the next slot, every position advanced by one.
-int encode_batch_step(gq8_batch *b)
+int encode_batch_step(gq8_batch *b, const gq8::RowsAttentionPlan &plan)
 {
     gq8_decoder *d = b->d;
     const gq8_shape &s = d->shape;
@@ -2274,12 +2283,12 @@ int encode_batch_step(gq8_batch *b)
         at.heads = s.heads;
         at.head_dim = s.head_dim;
         at.scale = 1.f / std::sqrt((float) s.head_dim);
-        at.per_split = gq8::rows_attention_split_keys(s.max_positions);
+        at.plan = plan;
         at.ws_o = b->attnO;
         at.ws_ml = b->attnMl;
         at.q8 = b->x8;
         at.q8_rows = S;
-        GQ8_STAGE(kStageAttention, gq8::launch_rows_attention(at, S, s.max_positions, st));
+        GQ8_STAGE(kStageAttention, gq8::launch_rows_attention(at, S, st));
         GQ8_BATCH_STAGE(kStageO, batch_product(b, d->qWidth, W, d->out[l],
                                                b->tiled ? b->tiledO[l] : nullptr, b->hidden, W, 1));
         GQ8_STAGE(kStageNorm, gq8::launch_rmsnorm(b->hidden, d->postNorm[l], S, W, s.rms_epsilon,
@@ -2317,15 +2326,15 @@ int encode_batch_step(gq8_batch *b)
     return GQ8_OK;
 }
 
-int ensure_batch_graph(gq8_batch *b)
+int ensure_batch_graph(gq8_batch *b, const gq8::RowsAttentionPlan &plan)
 {
-    if (b->graph)
+    if (b->graphs.count(plan.last_keys))
         return GQ8_OK;
     gq8_decoder *d = b->d;
     hipGraph_t graph = nullptr;
     GQ8_HIP(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
     d->capturing = true;
-    const int status = encode_batch_step(b);
+    const int status = encode_batch_step(b, plan);
     d->capturing = false;
     hipError_t end = hipStreamEndCapture(d->stream, &graph);
     if (status != GQ8_OK) {
@@ -2335,12 +2344,12 @@ int ensure_batch_graph(gq8_batch *b)
     }
     if (end != hipSuccess)
         return fail(GQ8_ERR_DEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(end));
-    hipError_t inst = hipGraphInstantiate(&b->graph, graph, nullptr, nullptr, 0);
+    hipGraphExec_t exec = nullptr;
+    hipError_t inst = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
     (void) hipGraphDestroy(graph);
-    if (inst != hipSuccess) {
-        b->graph = nullptr;
+    if (inst != hipSuccess)
         return fail(GQ8_ERR_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(inst));
-    }
+    b->graphs[plan.last_keys] = exec;
     return GQ8_OK;
 }
 
@@ -2360,8 +2369,8 @@ extern "C" void gq8_batch_destroy(gq8_batch *b)
         return;
     if (b->d && b->d->stream)
         (void) hipStreamSynchronize(b->d->stream);
-    if (b->graph)
-        (void) hipGraphExecDestroy(b->graph);
+    for (auto &g : b->graphs)
+        (void) hipGraphExecDestroy(g.second);
     for (void *p : b->allocations)
         (void) hipFree(p);
     delete b;
@@ -2525,13 +2534,15 @@ extern "C" int gq8_batch_decode(gq8_batch *b, int steps, int use_graph)
         return GQ8_OK;
     if (int st = refresh_tiled(b))
         return st;
-    if (use_graph)
-        if (int st = ensure_batch_graph(b))
-            return st;
+    if (use_graph) // every range's graph before the run, so no capture falls inside it
+        for (int i = 0; i < steps; ++i)
+            if (int st = ensure_batch_graph(b, batch_plan(b, i)))
+                return st;
     for (int i = 0; i < steps; ++i) {
+        const gq8::RowsAttentionPlan plan = batch_plan(b, i);
         if (use_graph)
-            GQ8_HIP(hipGraphLaunch(b->graph, b->d->stream));
-        else if (int st = encode_batch_step(b))
+            GQ8_HIP(hipGraphLaunch(b->graphs[plan.last_keys], b->d->stream));
+        else if (int st = encode_batch_step(b, plan))
             return st;
     }
     for (int &p : b->hostPositions)

@@ -706,58 +706,97 @@ __global__ __launch_bounds__(kThreads) void mqa_partial_kernel(
     }
 }
 
-// Merge: per query row, each split's maximum and sum rescaled to the row's
-// maximum, the factors computed once per (head, split) in LDS, the output
-// divided by the total, rounded to fp32 and optionally quantized.
+// Merge: a workgroup takes 512 channels of a query row, two a thread.  Lane s
+// of a wave holds split s's maximum and sum of a head, so the row's maximum,
+// the splits' factors and their total take a few lane exchanges, while the
+// first splits' channels are on their way; every split's channel is then
+// scaled and added in split order, divided by the total, rounded to fp32 and
+// optionally quantized.  (One workgroup a row, whose threads walked the 64
+// splits three times through memory, took 57 us for a row of 8000 keys.)
+// tiled: the rows' splits are launch_tiled_attention's (rows it finished
+// itself are left alone), else mqa_partial_kernel's.
+constexpr int kMergeBatch = 8;
+constexpr int kMergeChannels = 2 * kThreads;
+
 __global__ __launch_bounds__(kThreads) void mqa_merge_kernel(
     int heads, int head_dim, const int *pos_ptr, int pos_value, const double *__restrict__ ws_o,
-    const double *__restrict__ ws_ml, float *__restrict__ out, uint8_t *__restrict__ q8, int rows)
+    const double *__restrict__ ws_ml, float *__restrict__ out, uint8_t *__restrict__ q8, int rows,
+    int tiled, AttentionSplit split)
 {
-    __shared__ double sFactor[kMaxHeads * kMaxSplits];
-    __shared__ double sLargest[kMaxHeads], sTotal[kMaxHeads];
-    const int row = blockIdx.x;
-    const int keyCount = (pos_ptr ? *pos_ptr : 0) + pos_value + row + 1;
-    const int perSplit = keys_per_split(keyCount);
-    const int splits = (keyCount + perSplit - 1) / perSplit;
+    static_assert(kMaxSplits == 64, "a lane a split");
+    __shared__ double sFactor[kMaxHeads][kMaxSplits];
+    __shared__ double sTotal[kMaxHeads];
+    const int row = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int base = (pos_ptr ? *pos_ptr : 0) + pos_value;
+    int splits;
+    if (tiled) {
+        const int last = min((row / split.block_rows + 1) * split.block_rows, rows) - 1; // of the row's block
+        splits = tile_split((base + last) / kAttentionTileKeys + 1, split).splits;
+        if (splits == 1)
+            return;
+    } else {
+        const int keyCount = base + row + 1;
+        const int perSplit = keys_per_split(keyCount);
+        splits = (keyCount + perSplit - 1) / perSplit;
+    }
     const int qWidth = heads * head_dim;
-    const int64_t elements = (int64_t) rows * qWidth;
-    const double *ml = ws_ml + (int64_t) row * kMaxSplits * heads * 2;
+    const int first = blockIdx.x * kMergeChannels, end = min(first + kMergeChannels, qWidth);
+    const int h0 = first / head_dim, h1 = (end - 1) / head_dim;
+    const int64_t slot = (int64_t) row * kMaxSplits;
+    const double *o = ws_o + slot * qWidth;
+    int idx[2];
+    double part[2][kMergeBatch];
+    auto load = [&](int s0) {
+#pragma unroll
+        for (int s = 0; s < kMergeBatch; ++s)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) // clamped into range; not used past the ends
+                part[c][s] = o[(int64_t) min(s0 + s, splits - 1) * qWidth + min(idx[c], qWidth - 1)];
+    };
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+        idx[c] = first + c * kThreads + (int) threadIdx.x;
+    load(0);
 
-    if (threadIdx.x < heads) {
-        double largest = -INFINITY;
-        for (int s = 0; s < splits; ++s)
-            largest = fmax(largest, ml[((int64_t) s * heads + threadIdx.x) * 2]);
-        sLargest[threadIdx.x] = largest;
+    const bool live = lane < splits;
+    for (int h = h0 + wave; h <= h1; h += kThreads / 64) {
+        const double *ml = ws_ml + ((slot + (live ? lane : 0)) * heads + h) * 2;
+        const double m = live ? ml[0] : -INFINITY, sum = ml[1];
+        const double largest = wave_max(m);
+        // a split past the row's last key has m = -inf and weighs nothing
+        const double f = live ? exp(m - largest) : 0.0;
+        const double total = wave_sum(live ? sum * f : 0.0);
+        sFactor[h - h0][lane] = f;
+        if (lane == 0)
+            sTotal[h - h0] = total;
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < heads * splits; idx += kThreads) {
-        const int head = idx / splits, s = idx % splits;
-        sFactor[head * kMaxSplits + s] = exp(ml[((int64_t) s * heads + head) * 2] - sLargest[head]);
+    double weighted[2] = {0.0, 0.0};
+    int head[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+        head[c] = min(idx[c], qWidth - 1) / head_dim - h0;
+    for (int s0 = 0; s0 < splits; s0 += kMergeBatch) {
+        if (s0 > 0)
+            load(s0);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int s = 0; s < kMergeBatch; ++s)
+                if (s0 + s < splits)
+                    weighted[c] += part[c][s] * sFactor[head[c]][s0 + s];
     }
-    __syncthreads();
-    if (threadIdx.x < heads) {
-        double total = 0.0;
-        for (int s = 0; s < splits; ++s)
-            total += ml[((int64_t) s * heads + threadIdx.x) * 2 + 1]
-                     * sFactor[threadIdx.x * kMaxSplits + s];
-        sTotal[threadIdx.x] = total;
-    }
-    __syncthreads();
-
-    const double *o = ws_o + (int64_t) row * kMaxSplits * qWidth;
-    for (int idx = threadIdx.x; idx < qWidth; idx += kThreads) {
-        const int head = idx / head_dim;
-        const double *factor = sFactor + head * kMaxSplits;
-        double weighted = 0.0;
-        for (int s = 0; s < splits; ++s)
-            weighted += o[(int64_t) s * qWidth + idx] * factor[s];
-        const float v = (float) (weighted / sTotal[head]);
-        const int64_t at = (int64_t) row * qWidth + idx;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        if (idx[c] >= qWidth) // whole 32-lane groups where there is a q8
+            continue;
+        const float v = (float) (weighted[c] / sTotal[head[c]]);
+        const int64_t at = (int64_t) row * qWidth + idx[c];
         if (out)
             out[at] = v;
         if (q8)
-            quantize_in_group(v, threadIdx.x & 31, q8 + at,
-                              reinterpret_cast<uint16_t *>(q8 + elements) + at / kBlock);
+            quantize_in_group(v, lane & 31, q8 + at,
+                              reinterpret_cast<uint16_t *>(q8 + (int64_t) rows * qWidth) + at / kBlock);
     }
 }
 
@@ -1099,20 +1138,32 @@ hipError_t launch_mqa(const float *queries, int q_stride, const uint16_t *key_ca
         return hipErrorInvalidValue;
     if (q8 && (heads * head_dim) % kBlock != 0)
         return hipErrorInvalidValue;
-    if (rows >= kPrefillAttentionMinRows
-        && prefill_attention_supported(head_dim, queries, q_stride, key_cache, value_cache, out, q8))
-        return launch_prefill_attention(queries, q_stride, key_cache, value_cache, heads, kv_heads,
-                                        head_dim, rows, pos_ptr, pos_value, scale, out, q8, stream);
     double *wsO = reinterpret_cast<double *>(workspace);
     double *wsMl = wsO + (int64_t) rows * kMaxSplits * heads * head_dim;
-    hipLaunchKernelGGL(mqa_partial_kernel, dim3(kMaxSplits, rows), dim3(kThreads), 0, stream,
-                       queries, q_stride, key_cache, value_cache, heads, kv_heads, head_dim,
-                       pos_ptr, pos_value, scale, wsO, wsMl);
-    hipError_t status = hipGetLastError();
-    if (status != hipSuccess)
-        return status;
-    hipLaunchKernelGGL(mqa_merge_kernel, dim3(rows), dim3(kThreads), 0, stream, heads, head_dim,
-                       pos_ptr, pos_value, wsO, wsMl, out, q8, rows);
+    const bool tiled = tiled_attention_supported(head_dim, queries, q_stride, key_cache, value_cache,
+                                                 out, q8);
+    AttentionSplit split{1, 4, 1};
+    bool merges = true;
+    if (tiled) {
+        split = attention_split(rows, heads, kv_heads, pos_ptr ? 0 : pos_value + rows);
+        hipError_t status = launch_tiled_attention(queries, q_stride, key_cache, value_cache, heads,
+                                                   kv_heads, head_dim, rows, pos_ptr, pos_value,
+                                                   scale, out, q8, split, wsO, wsMl, stream);
+        if (status != hipSuccess)
+            return status;
+        merges = pos_ptr || tile_split((pos_value + rows - 1) / kAttentionTileKeys + 1, split).splits > 1;
+    } else {
+        hipLaunchKernelGGL(mqa_partial_kernel, dim3(kMaxSplits, rows), dim3(kThreads), 0, stream,
+                           queries, q_stride, key_cache, value_cache, heads, kv_heads, head_dim,
+                           pos_ptr, pos_value, scale, wsO, wsMl);
+        hipError_t status = hipGetLastError();
+        if (status != hipSuccess)
+            return status;
+    }
+    if (merges)
+        hipLaunchKernelGGL(mqa_merge_kernel, dim3(blocks_for(heads * head_dim, kMergeChannels), rows),
+                           dim3(kThreads), 0, stream, heads, head_dim, pos_ptr, pos_value, wsO, wsMl, out, q8, rows,
+                           tiled ? 1 : 0, split);
     return hipGetLastError();
 }
 

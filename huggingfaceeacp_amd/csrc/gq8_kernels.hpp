@@ -70,18 +70,41 @@ constexpr int kMaxHeadDim = 256;
 
 size_t mqa_workspace_bytes(int rows, int heads, int head_dim, int max_keys);
 
-// Blocks of kPrefillAttentionMinRows rows or more with a head width of 64, 128
-// or 256 take the fp64-MFMA prefill kernel (gq8_prefill_attention.hip; no
-// workspace) when its 16-byte loads and stores fit the buffers: queries, caches,
-// out and q8 16-byte aligned, q_stride a multiple of 4.
-constexpr int kPrefillAttentionMinRows = 16;
-bool prefill_attention_supported(int head_dim, const float *queries, int q_stride,
-                                 const uint16_t *key_cache, const uint16_t *value_cache,
-                                 const float *out, const uint8_t *q8);
-hipError_t launch_prefill_attention(const float *queries, int q_stride, const uint16_t *key_cache,
-                                    const uint16_t *value_cache, int heads, int kv_heads,
-                                    int head_dim, int rows, const int *pos_ptr, int pos_value,
-                                    float scale, float *out, uint8_t *q8, hipStream_t stream);
+// How the tiled attention (gq8_prefill_attention.hip) splits a step: blocks
+// of block_rows query rows, each block's key tiles over workgroups of `tiles`
+// tiles (whole rounds of a workgroup's four waves; more where a block would
+// need over max_splits of them).
+constexpr int kAttentionTileKeys = 16;
+struct AttentionSplit {
+    int block_rows, tiles, max_splits;
+};
+// A block of `tiles` key tiles: `splits` workgroups, `per` tiles each (the last
+// may hold fewer).
+struct TileSplit {
+    int splits, per;
+};
+__host__ __device__ inline TileSplit tile_split(int tiles, const AttentionSplit &s)
+{
+    const int least = ((tiles + s.max_splits - 1) / s.max_splits + 3) / 4 * 4;
+    const int per = least > s.tiles ? least : s.tiles;
+    return {(tiles + per - 1) / per, per};
+}
+// keys: what the last row attends, 0 where only the device knows.
+AttentionSplit attention_split(int rows, int heads, int kv_heads, int keys);
+
+// The fp64-MFMA attention takes head widths of 64, 128 and 256 when its 16-byte
+// loads and stores fit the buffers: queries, caches, out and q8 16-byte aligned,
+// q_stride a multiple of 4.  Blocks in one workgroup finish their rows; the
+// splits of the others leave ws_o / ws_ml (launch_mqa's workspace) for its
+// merge.
+bool tiled_attention_supported(int head_dim, const float *queries, int q_stride,
+                               const uint16_t *key_cache, const uint16_t *value_cache,
+                               const float *out, const uint8_t *q8);
+hipError_t launch_tiled_attention(const float *queries, int q_stride, const uint16_t *key_cache,
+                                  const uint16_t *value_cache, int heads, int kv_heads,
+                                  int head_dim, int rows, const int *pos_ptr, int pos_value,
+                                  float scale, float *out, uint8_t *q8, const AttentionSplit &split,
+                                  double *ws_o, double *ws_ml, hipStream_t stream);
 
 // Rows of queries (row stride q_stride) at positions base + r where
 // base = (*pos_ptr if pos_ptr) + pos_value; row r attends keys [0, base + r].

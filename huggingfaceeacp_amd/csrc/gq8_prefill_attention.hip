@@ -7,15 +7,23 @@
 // kernel and the oracle; the block's rows leave as fp32 and as the Q8 row of
 // the o product.
 //
-// Work split: a workgroup owns 16 consecutive rows of one head; its four
-// waves take the key tiles (16 keys) round robin, each keeping an online
-// softmax state (row maximum, sum and the 16 x head_dim sums), and the states
-// are merged in LDS at the end.  The grid starts the longest row blocks
-// first, so the short ones fill in behind them.  A wave requests a tile's
-// values (16-byte loads) before its scores and the next tile's keys right
-// after them, so no tile's operands wait in registers a whole tile ahead; the
-// kernel is held to two waves a SIMD (256 registers a wave), and one wave's
-// MFMAs run while the other waits on its loads or works on its softmax.
+// Work split: the query heads of one KV head and position share their keys, so
+// a workgroup owns 16 (row, head) pairs of one KV head: block_rows consecutive
+// rows with all of the KV head's query heads (two rows at eight heads a KV
+// head).  Fewer than 16 rows take one row a block, so no row's arithmetic
+// meets another row's keys.  The block's key tiles (16 keys) are split over
+// several workgroups where the blocks alone would leave the chip idle or end
+// unevenly (split_plan); a workgroup's four waves take its tiles round robin,
+// each keeping an online softmax state (row maximum, sum and the 16 x head_dim
+// sums), and the states are merged in LDS at the end.  A block in one
+// workgroup finishes its rows there; the splits of one leave their scaled sums,
+// maxima and totals in the workspace for the merge launch.  The grid starts the
+// longest blocks first, so the short ones fill in behind them.  A wave
+// requests a tile's values (16-byte loads) before its scores and the next
+// tile's keys right after them, so no tile's operands wait in registers a
+// whole tile ahead; the kernel is held to two waves a SIMD (256 registers a
+// wave), and one wave's MFMAs run while the other waits on its loads or works
+// on its softmax.
 //
 // Per tile a wave computes S^T = K Q^T with v_mfma_f64_16x16x4f64, so the
 // result holds row j of the block on lanes j, j + 16, j + 32, j + 48 and is
@@ -40,12 +48,15 @@
 #include "gq8_kernels.hpp"
 #include "gq8_numerics.hpp"
 
+#include <algorithm>
+#include <cmath>
+
 namespace gq8 {
 namespace {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-constexpr int kPaRows = 16;   // query rows a workgroup
+constexpr int kPaRows = 16;   // (row, head) pairs a workgroup
 constexpr int kPaWaves = 4;
 constexpr int kPaThreads = kPaWaves * 64;
 constexpr int kPaKeys = 16;   // keys a tile
@@ -62,6 +73,8 @@ struct PrefillArgs {
     float scale;
     float *out;   // optional [rows, heads * head_dim]
     uint8_t *q8;  // optional Q8 row buffer of rows x heads * head_dim
+    AttentionSplit split;
+    double *ws_o, *ws_ml; // the splits' sums and (maximum, total)s (mqa_merge_kernel's layout)
 };
 
 __device__ inline v4d mfma(double a, double b, v4d c)
@@ -92,8 +105,13 @@ __device__ inline double half_at(const uint32_t (&w)[N], int i)
     return (double) half_value((uint16_t) (w[i >> 1] >> (16 * (i & 1))));
 }
 
-// E channels a lane group, T = head_dim / 16 output column tiles.
-template <int E>
+// E channels a lane group, T = head_dim / 16 output column tiles.  kOneRow:
+// blocks of one query row, whose every attended key is its own (a step of few
+// rows): the copies of the last key in the last tile are zeroed there, since a
+// zero weight times an infinity would not be zero.  Blocks of several rows
+// read later rows' keys under a zero weight in any case, and do without the
+// selects (2-3 % of the kernel).
+template <int E, bool kOneRow>
 __global__ __launch_bounds__(kPaThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_attention_kernel(PrefillArgs a)
 {
@@ -114,26 +132,31 @@ void prefill_attention_kernel(PrefillArgs a)
 
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int g = lane >> 4, j = lane & 15;
-    const int blocks = (a.rows + kPaRows - 1) / kPaRows;
-    const int rb = blocks - 1 - (int) blockIdx.x / a.heads; // the longest row blocks first
-    const int h = (int) blockIdx.x % a.heads;
-    const int r0 = rb * kPaRows;
+    const int perKv = a.heads / a.kv_heads, blockRows = a.split.block_rows;
+    const int blocks = (a.rows + blockRows - 1) / blockRows;
+    const int rb = blocks - 1 - (int) blockIdx.x / a.kv_heads; // the longest blocks first
+    const int kvh = (int) blockIdx.x % a.kv_heads;
+    const int r0 = rb * blockRows;
     const int qWidth = a.heads * HD, kvWidth = a.kv_heads * HD;
-    const int kvh = h / (a.heads / a.kv_heads);
     const int base = (a.pos_ptr ? *a.pos_ptr : 0) + a.pos_value;
-    const int rowsHere = min(kPaRows, a.rows - r0);
+    const int rowsHere = min(blockRows, a.rows - r0);
+    const int pairs = rowsHere * perKv;            // pair p: row r0 + p / perKv, head p % perKv of the KV head
     const int lastKey = base + r0 + rowsHere - 1;  // the block's last row attends [0, lastKey]
-    const int tiles = lastKey / kPaKeys + 1;
-    const int myRow = min(j, rowsHere - 1);        // rows past the block repeat its last row
-    const int rowPos = base + r0 + myRow;
+    const TileSplit span = tile_split(lastKey / kPaKeys + 1, a.split);
+    if ((int) blockIdx.y >= span.splits)
+        return;
+    const int firstTile = (int) blockIdx.y * span.per;
+    const int tiles = min(firstTile + span.per, lastKey / kPaKeys + 1); // this split's end
+    const int rowPos = base + r0 + min(j, pairs - 1) / perKv; // pairs past the block repeat its last
 
-    // the block's query rows in LDS (rows past the block repeat its last row);
-    // lane (g, j) reads row j's channels [g E, g E + E), the B operand of S^T
+    // the block's query rows in LDS (pairs past the block repeat its last);
+    // lane (g, j) reads pair j's channels [g E, g E + E), the B operand of S^T
 #pragma unroll
     for (int i = t; i < kPaRows * HD / 4; i += kPaThreads) {
-        const int row = i / (HD / 4), c = (i % (HD / 4)) * 4;
-        const float *src = a.queries + (int64_t) (r0 + min(row, rowsHere - 1)) * a.q_stride + h * HD + c;
-        *reinterpret_cast<float4 *>(&sQ[row][c]) = *reinterpret_cast<const float4 *>(src);
+        const int pair = min(i / (HD / 4), pairs - 1), c = (i % (HD / 4)) * 4;
+        const float *src = a.queries + (int64_t) (r0 + pair / perKv) * a.q_stride
+                           + (kvh * perKv + pair % perKv) * HD + c;
+        *reinterpret_cast<float4 *>(&sQ[i / (HD / 4)][c]) = *reinterpret_cast<const float4 *>(src);
     }
     __syncthreads();
     const int qAt = j * (HD + 4) + g * E; // lane (g, j)'s first query channel in sQ
@@ -159,9 +182,9 @@ void prefill_attention_kernel(PrefillArgs a)
         o[n] = v4d{0.0, 0.0, 0.0, 0.0};
 
     uint32_t kw[KW], vw[4][VW];
-    if (wave < tiles)
-        load_keys(wave, kw);
-    for (int tile = wave; tile < tiles; tile += kPaWaves) {
+    if (firstTile + wave < tiles)
+        load_keys(firstTile + wave, kw);
+    for (int tile = firstTile + wave; tile < tiles; tile += kPaWaves) {
         load_values(tile, vw); // arrive while the scores are computed
         const int k0 = tile * kPaKeys;
 
@@ -222,6 +245,14 @@ void prefill_attention_kernel(PrefillArgs a)
         sum += __shfl_xor(sum, 32);
         l += sum;
 
+        if (kOneRow && k0 + kPaKeys - 1 > lastKey) {
+#pragma unroll
+            for (int st = 0; st < 4; ++st)
+#pragma unroll
+                for (int w = 0; w < VW; ++w)
+                    vw[st][w] = k0 + g + 4 * st <= lastKey ? vw[st][w] : 0u;
+        }
+
         // O += P V, four keys a step
 #pragma unroll
         for (int st = 0; st < 4; ++st)
@@ -240,9 +271,8 @@ void prefill_attention_kernel(PrefillArgs a)
     }
 
     // merge the waves' states.  Every wave scales its sums to the rows'
-    // common maximum (wave 0 holds tile 0, which every row attends, so that
-    // maximum is finite; a wave whose keys a row never reached has m = -inf
-    // and weighs nothing); then the waves exchange their sums kMergeTiles
+    // common maximum (a wave whose keys a row never reached has m = -inf and
+    // weighs nothing; in a split past a row's last key every wave has); then the waves exchange their sums kMergeTiles
     // column tiles at a time, and wave w adds the four waves' sums of its
     // rows g + 4 w in wave order and finishes those rows.
 #pragma unroll
@@ -287,12 +317,33 @@ void prefill_attention_kernel(PrefillArgs a)
     for (int w = 1; w < kPaWaves; ++w)
         total += sSum[w][wave][lane];
 
-    // row g + 4 wave, channels [j T, j T + T): fp32, then Q8 per 32-block
-    // (kBlockLanes neighbouring lanes a block)
+    // pair g + 4 wave, channels [j T, j T + T)
     {
-        const int row = g + 4 * wave;
-        const bool live = row < rowsHere;
-        const int64_t at = (int64_t) (r0 + min(row, rowsHere - 1)) * qWidth + h * HD + j * T;
+        const int pair = g + 4 * wave;
+        const bool live = pair < pairs;
+        const int row = r0 + min(pair, pairs - 1) / perKv;
+        const int head = kvh * perKv + min(pair, pairs - 1) % perKv;
+        const int64_t at = (int64_t) row * qWidth + head * HD + j * T;
+        if (span.splits > 1) { // one of several: its sums, maximum and total for the merge
+            if (!live)
+                return;
+            double common = sMax[0][wave][lane];
+#pragma unroll
+            for (int w = 1; w < kPaWaves; ++w)
+                common = fmax(common, sMax[w][wave][lane]);
+            const int64_t slot = (int64_t) row * kAttentionSplits + blockIdx.y;
+            double *o = a.ws_o + slot * qWidth + head * HD + j * T;
+#pragma unroll
+            for (int n = 0; n < T; ++n)
+                o[n] = mine[n];
+            if (j == 0) {
+                a.ws_ml[(slot * a.heads + head) * 2] = common;
+                a.ws_ml[(slot * a.heads + head) * 2 + 1] = total;
+            }
+            return;
+        }
+        // the whole row: fp32, then Q8 per 32-block (kBlockLanes neighbouring
+        // lanes a block)
         float v[T];
         float amax = 0.f;
 #pragma unroll
@@ -339,7 +390,7 @@ void prefill_attention_kernel(PrefillArgs a)
 
 } // namespace
 
-bool prefill_attention_supported(int head_dim, const float *queries, int q_stride,
+bool tiled_attention_supported(int head_dim, const float *queries, int q_stride,
                                  const uint16_t *key_cache, const uint16_t *value_cache,
                                  const float *out, const uint8_t *q8)
 {
@@ -349,29 +400,105 @@ bool prefill_attention_supported(int head_dim, const float *queries, int q_strid
            && aligned(q8);
 }
 
-hipError_t launch_prefill_attention(const float *queries, int q_stride, const uint16_t *key_cache,
-                                    const uint16_t *value_cache, int heads, int kv_heads,
-                                    int head_dim, int rows, const int *pos_ptr, int pos_value,
-                                    float scale, float *out, uint8_t *q8, hipStream_t stream)
+// The split with the least estimated time.  A workgroup keeps a compute
+// unit's matrix cores about as busy as two do (5.3 us a round of four tiles
+// alone, 10.6 each beside another), so a unit is taken to run its workgroups
+// one after another, the fullest unit ending last; the merge launch and the
+// partials cost some microseconds and more with the rows.  Within 10 % of most
+// of a sweep at eight heads of 256 over one KV head (rows 1 .. 2048, 0 .. 8000
+// keys before them).  Microseconds there, one workgroup a block -> split: 333
+// rows behind 700 keys 99 -> 77, 128 behind 4000 352 -> 105, 16 behind 8000
+// 672 -> 42, one row of 8000 keys 680 -> 31 (110 in mqa_partial_kernel and its
+// former merge); 512 rows behind 512 keys and 2048 alone stay whole (94, 330).
+AttentionSplit attention_split(int rows, int heads, int kv_heads, int keys)
+{
+    constexpr int kUnits = 256, kSamples = 32;
+    constexpr double kRound = 5.3, kStart = 5.0, kMerge = 4.0, kMergeRow = 0.012;
+    constexpr double kWorth = 0.92; // a split's estimate against the whole blocks'
+    AttentionSplit s{rows < kPaRows ? 1 : std::max(1, kPaRows / (heads / kv_heads)), 8,
+                     kAttentionSplits};
+    if (keys <= 0)
+        return s;
+    if (rows > 65535) { // past the merge's grid
+        s.max_splits = 1;
+        return s;
+    }
+    const int blocks = (rows + s.block_rows - 1) / s.block_rows;
+    auto block_tiles = [&](int b) { // key tiles of block b
+        return (keys - rows + std::min((b + 1) * s.block_rows, rows) - 1) / kAttentionTileKeys + 1;
+    };
+    const int longest = block_tiles(blocks - 1);
+    const int stride = (blocks + kSamples - 1) / kSamples, samples = (blocks + stride - 1) / stride;
+    double least = 0.0;
+    int chosen = 0;
+    for (int splits = 1, last = 0; splits <= kAttentionSplits; splits += 1 + splits / 4) {
+        const int per = ((longest + splits - 1) / splits + 3) / 4 * 4;
+        if (per == last)
+            continue;
+        last = per;
+        // the sampled blocks' workgroups and rounds of four tiles
+        int64_t count = 0, rounds = 0;
+        int smallest = per;
+        for (int b = blocks - 1; b >= 0; b -= stride) {
+            const int tiles = block_tiles(b), whole = tiles / per, rest = tiles % per;
+            count += whole + (rest ? 1 : 0);
+            rounds += whole * (per / 4) + (rest + 3) / 4;
+            smallest = std::min(smallest, whole ? per : rest);
+        }
+        const double each = (double) blocks * kv_heads / samples / kUnits; // a unit's share of a sample
+        const double mine = count * each;
+        // the fullest unit: the longest workgroup, or its share of all rounds
+        // and what whole workgroups leave uneven (the short ones go last)
+        const double longestOne = (std::min(per, longest) + 3) / 4;
+        const double busy = std::max(longestOne, rounds * each + (std::ceil(mine) - mine) * (smallest + 3) / 4);
+        const double cost = busy * kRound + std::ceil(mine) * kStart
+                            + (longest > per ? kMerge + rows * kMergeRow : 0.0);
+        if (chosen == 0 || cost < least) {
+            least = chosen == 0 ? kWorth * cost : cost;
+            chosen = per;
+        }
+    }
+    s.tiles = chosen;
+    return s;
+}
+
+hipError_t launch_tiled_attention(const float *queries, int q_stride, const uint16_t *key_cache,
+                                  const uint16_t *value_cache, int heads, int kv_heads,
+                                  int head_dim, int rows, const int *pos_ptr, int pos_value,
+                                  float scale, float *out, uint8_t *q8, const AttentionSplit &split,
+                                  double *ws_o, double *ws_ml, hipStream_t stream)
 {
     if (rows <= 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0
-        || !prefill_attention_supported(head_dim, queries, q_stride, key_cache, value_cache, out, q8)
-        || q_stride < heads * head_dim)
+        || heads / kv_heads > kPaRows
+        || !tiled_attention_supported(head_dim, queries, q_stride, key_cache, value_cache, out, q8)
+        || q_stride < heads * head_dim || split.block_rows <= 0
+        || split.block_rows * (heads / kv_heads) > kPaRows || split.max_splits <= 0
+        || split.max_splits > kAttentionSplits || split.tiles <= 0 || split.tiles % kPaWaves != 0
+        || (split.max_splits > 1 && (!ws_o || !ws_ml)))
         return hipErrorInvalidValue;
     PrefillArgs a{queries, q_stride, key_cache, value_cache, heads, kv_heads, head_dim, rows,
-                  pos_ptr, pos_value, scale, out, q8};
-    const dim3 grid((unsigned) ((rows + kPaRows - 1) / kPaRows * heads));
+                  pos_ptr, pos_value, scale, out, q8, split, ws_o, ws_ml};
+    const int blocks = (rows + split.block_rows - 1) / split.block_rows;
+    // the splits of the longest block, where its keys are known here and every
+    // block's workgroups take the same tiles
+    const TileSplit longest = tile_split((pos_value + rows - 1) / kPaKeys + 1, split);
+    const int splits = pos_ptr || longest.per != split.tiles ? split.max_splits : longest.splits;
+    const dim3 grid((unsigned) (blocks * kv_heads), splits);
+#define GQ8_TILED_ATTENTION(E)                                                                  \
+    do {                                                                                       \
+        if (split.block_rows == 1)                                                             \
+            hipLaunchKernelGGL((prefill_attention_kernel<E, true>), grid, dim3(kPaThreads), 0,   \
+                               stream, a);                                                     \
+        else                                                                                   \
+            hipLaunchKernelGGL((prefill_attention_kernel<E, false>), grid, dim3(kPaThreads), 0,  \
+                               stream, a);                                                     \
+    } while (0)
     switch (head_dim) {
-    case 256:
-        hipLaunchKernelGGL(prefill_attention_kernel<64>, grid, dim3(kPaThreads), 0, stream, a);
-        break;
-    case 128:
-        hipLaunchKernelGGL(prefill_attention_kernel<32>, grid, dim3(kPaThreads), 0, stream, a);
-        break;
-    default:
-        hipLaunchKernelGGL(prefill_attention_kernel<16>, grid, dim3(kPaThreads), 0, stream, a);
-        break;
+    case 256: GQ8_TILED_ATTENTION(64); break;
+    case 128: GQ8_TILED_ATTENTION(32); break;
+    default: GQ8_TILED_ATTENTION(16); break;
     }
+#undef GQ8_TILED_ATTENTION
     return hipGetLastError();
 }
 

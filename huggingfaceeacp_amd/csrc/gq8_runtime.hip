@@ -1608,6 +1608,11 @@ int encode_step(gq8_decoder *d, int rows, float *logits, int logitsRows, bool sa
     const bool dbg = d->debug;
     if (rows == 1 && logits && logitsRows == 1 && d->useFused && d->fusedSupported)
         return encode_fused_token(d, logits, sample);
+    // A step that is not captured runs at the host's position (steps are
+    // enqueued in order), so the attention can be split by its keys; a
+    // captured one reads the device's.
+    const int *devicePosition = d->capturing ? d->position : nullptr;
+    const int hostPosition = d->capturing ? 0 : d->hostPosition;
 
     GQ8_STAGE(kStageEmbed, gq8::launch_embed(d->sequence, d->position, rows, d->embedding, s.vocab, W,
                                  s.embedding_scale, d->hidden, st));
@@ -1627,7 +1632,7 @@ int encode_step(gq8_decoder *d, int rows, float *logits, int logitsRows, bool sa
                                        d->position, 0, rows, d->cosines, d->sines, keys, values,
                                        st));
         GQ8_STAGE(kStageAttention, gq8::launch_mqa(d->qkvRows, d->qkvWidth, keys, values, s.heads, s.kv_heads,
-                                   s.head_dim, rows, d->position, 0, s.max_positions,
+                                   s.head_dim, rows, devicePosition, hostPosition, s.max_positions,
                                    attentionScale, dbg ? d->debugAttended : nullptr, d->x8,
                                    d->attentionWorkspace, d->attentionWorkspaceBytes, st));
         if (dbg && capture_debug(d, 1, l, d->debugAttended, rows, d->qWidth, d->x8))

@@ -229,9 +229,10 @@ struct SampleArgs {
     float temperature;     // > 0 (zero is the argmax)
     int top_k;             // 0: no cut
     float top_p;           // 1: no cut
-    const double *draws;   // uniform draws in [0, 1), one a sample
+    const double *draws;   // uniform draws in [0, 1), one a sample (null: `uniform`)
     int draw_count;        // the index is clamped to the last draw
     int *draw_index;       // the draw this sample takes; advanced by one
+    double uniform;        // the draw where there are no draws
     uint32_t *sequence;    // the chosen id goes to sequence[*position + offset] (optional)
     const int *position;
     int offset;

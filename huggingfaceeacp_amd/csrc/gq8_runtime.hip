@@ -475,8 +475,7 @@ extern "C" size_t gq8_argmax_workspace_bytes(int rows, int length)
 
 extern "C" size_t gq8_sample_workspace_bytes(int vocab)
 {
-    // the sort's buffers, then one draw and its index
-    return vocab > 0 ? std::max(gq8::sample_workspace_bytes(vocab) + 256,
+    return vocab > 0 ? std::max(gq8::sample_workspace_bytes(vocab),
                                 gq8::argmax_workspace_bytes(1, vocab))
                      : 0;
 }
@@ -501,15 +500,6 @@ extern "C" int gq8_sample_row(const float *logits, const float *mask, int vocab,
                                       gq8::argmax_workspace_bytes(1, vocab), st));
         return GQ8_OK;
     }
-    const size_t sortBytes = gq8::sample_workspace_bytes(vocab);
-    auto *tail = reinterpret_cast<uint8_t *>(workspace) + sortBytes;
-    auto *draw = reinterpret_cast<double *>(tail);
-    auto *index = reinterpret_cast<int *>(tail + sizeof(double));
-    struct {
-        double u;
-        int index;
-    } host{uniform, 0};
-    GQ8_HIP(hipMemcpyAsync(draw, &host, sizeof(host), hipMemcpyHostToDevice, st));
     gq8::SampleArgs a{};
     a.logits = logits;
     a.mask = mask;
@@ -517,12 +507,9 @@ extern "C" int gq8_sample_row(const float *logits, const float *mask, int vocab,
     a.temperature = options->temperature;
     a.top_k = options->top_k;
     a.top_p = options->top_p;
-    a.draws = draw;
-    a.draw_count = 1;
-    a.draw_index = index;
+    a.uniform = uniform;
     a.token_out = token;
-    GQ8_LAUNCH(gq8::launch_sample(a, workspace, sortBytes, st));
-    // the draw is read from host memory that ends with this call
+    GQ8_LAUNCH(gq8::launch_sample(a, workspace, gq8::sample_workspace_bytes(vocab), st));
     GQ8_HIP(hipStreamSynchronize(st));
     return GQ8_OK;
 }

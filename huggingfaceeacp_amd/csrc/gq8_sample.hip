@@ -3,19 +3,37 @@
 // readback (Gemma.cpp:545-595).
 //
 // Candidates are the unmasked tokens, scored logit * (1 / temperature) in
-// double.  With top-k or top-p they are ranked (score descending, token
-// ascending) by a stable LSD radix sort of a 64-bit order key over the
-// token-ordered row: eight passes of an 8-bit digit, each a histogram, a scan
-// and a scatter that places every element by its rank among equal digits
-// (wave ballots, then wave and round prefixes in LDS), so ties keep token
-// order exactly as the reference's comparison does.  One workgroup then
-// walks the ranked candidates (or the row in token order when no cut is set,
-// as the reference's draw does): the softmax over the survivors, the top-p
-// prefix whose running mass reaches p (boundary kept), and the first
-// candidate whose running mass passes the draw.  Running sums go a contiguous
-// chunk a thread and then chunk by chunk in order, so only the rounding of
-// the sums differs from the reference's sequential loop.  The uniform draws
-// come from the caller (the top 53 bits of std::mt19937_64 outputs).
+// double and weighing exp(score - largest score).  With a cut set they are
+// ranked (score descending, token ascending): the first k are kept, of those
+// the shortest prefix whose mass reaches p of theirs, and the draw takes the
+// first candidate whose running mass passes uniform of what is left.  With
+// no cut the draw walks the row in token order, as the reference's does.
+//
+// Nothing sorts the row.  Each step needs one place in the ranking (the k-th
+// candidate, the one that reaches a mass), so the row is spread over 2048
+// bins of the distance to the largest score, whose order is the ranking's; a
+// scan of the bins' counts and masses gives the bin that holds the place, and
+// that bin's candidates alone are ranked.  A bin past kRankCap candidates is
+// spread over 2048 bins again, of the range its (score, token) keys cover,
+// until few enough are left, so a flat row or one of equal logits costs a few
+// passes over its own candidates.  Four launches:
+//   sample_max_kernel      each chunk's largest score, unmasked count and last
+//                          unmasked token; the bins cleared
+//   sample_bins_kernel     the chunks' masses; the bins' counts and masses
+//   sample_gather_kernel   the candidates of the bins that a cut can reach,
+//                          bin after bin
+//   sample_draw_kernel     one workgroup: the cuts and the draw
+// A bin's mass is summed as integers of 2^-32 and 2^-64, so it does not depend
+// on the order the atomics land in (and is within 2^-65 a candidate of exact);
+// the sums along the ranking are doubles, so only their rounding differs from
+// the reference's sequential loop.  The uniform draws come from the caller
+// (the top 53 bits of std::mt19937_64 outputs).
+//
+// The launches are bound by their chains (a read of the chunk's 16 KB, the
+// atomics, the scans), not by the row's 1 MB.  A row of 256 000 normal logits
+// (sigma 3) at temperature 0.8, top-k 40, top-p 0.95: 69 us; the eight-pass
+// radix sort of the row, its one-workgroup scans and the draw over the ranked
+// row had taken 811.
 #include "gq8_device.hpp"
 #include "gq8_kernels.hpp"
 #include "gq8_numerics.hpp"
@@ -26,22 +44,36 @@
 namespace gq8 {
 namespace {
 
-constexpr int kSortThreads = 256;
-constexpr int kSortRounds = 8;                          // elements a thread a tile
-constexpr int kSortTile = kSortThreads * kSortRounds;   // 2048
-constexpr int kDrawThreads = 1024;
-constexpr uint64_t kMaskedKey = ~0ull;
+constexpr int kSampleThreads = 1024;
+constexpr int kSampleWaves = kSampleThreads / 64;
+constexpr int kChunkRounds = 4;                                // tokens a thread
+constexpr int kChunkTokens = kSampleThreads * kChunkRounds;    // 4096 a workgroup
+constexpr int kBins = 2 * kSampleThreads;                      // two a thread in the scans
+constexpr int kRankCap = 512;                                  // candidates ranked by counting
 
-struct SampleWorkspace {
-    uint64_t *keys[2];
-    uint32_t *tokens[2];
-    int *hist; // [256][tiles]
-    int tiles;
+struct ChunkState {
+    double largest; // of the chunk's unmasked scores, -DBL_MAX where there is none
+    double mass;    // of its weights, in a fixed order
+    int count;      // unmasked tokens
+    int last;       // the last of them, -1 where there is none
+    int bad;        // a NaN or +infinite logit among them: no sum of weights is a number
+    int unused;
 };
 
-int sort_tiles(int vocab)
+struct SampleWorkspace {
+    ChunkState *chunks;
+    ChunkState *row;    // the whole row's
+    uint32_t *counts;   // of the bins
+    uint32_t *cursors;  // candidates of a bin gathered so far
+    uint64_t *massHi;   // multiples of 2^-32
+    uint64_t *massLo;   // multiples of 2^-64
+    uint64_t *gathered; // (ranking key, token), bin after bin
+    int chunkCount;
+};
+
+int sample_chunks(int vocab)
 {
-    return (vocab + kSortTile - 1) / kSortTile;
+    return (vocab + kChunkTokens - 1) / kChunkTokens;
 }
 
 size_t align256(size_t n)
@@ -49,293 +81,700 @@ size_t align256(size_t n)
     return (n + 255) & ~size_t(255);
 }
 
-// Scores: +0 for a zero (the reference compares scores by value, so -0 and +0
-// tie), the order key descending in score.
+// +0 for a zero (the reference compares scores by value, so -0 and +0 tie)
 __device__ inline double candidate_score(float logit, double inverse)
 {
     const double s = (double) logit * inverse;
     return s == 0.0 ? 0.0 : s;
 }
 
-__device__ inline uint64_t descending_key(double s)
+// The ranking key of a candidate: descending in the logit (the score is
+// strictly increasing in it), then ascending in the token.
+__device__ inline uint64_t ranking_key(float logit, uint32_t token)
 {
-    uint64_t u = (uint64_t) __double_as_longlong(s);
-    u = (u >> 63) ? ~u : (u | (1ull << 63));
-    return ~u;
+    uint32_t u = __float_as_uint(logit == 0.f ? 0.f : logit);
+    u = (u >> 31) ? ~u : (u | (1u << 31));
+    return ((uint64_t) ~u << 32) | token;
 }
 
-__device__ inline double score_of_key(uint64_t key)
+__device__ inline float logit_of_key(uint64_t key)
 {
-    uint64_t u = ~key;
-    u = (u >> 63) ? (u & ~(1ull << 63)) : ~u;
-    return __longlong_as_double((long long) u);
+    uint32_t u = ~(uint32_t) (key >> 32);
+    u = (u >> 31) ? (u & ~(1u << 31)) : ~u;
+    return __uint_as_float(u);
 }
 
-__global__ __launch_bounds__(kSortThreads) void sample_keys_kernel(SampleArgs a, uint64_t *keys,
-                                                                   uint32_t *tokens)
+__device__ inline double candidate_weight(float logit, double inverse, double top)
 {
-    const double inverse = 1.0 / (double) a.temperature;
-    for (int r = 0; r < kSortRounds; ++r) {
-        const int e = blockIdx.x * kSortTile + r * kSortThreads + threadIdx.x;
-        if (e >= a.vocab)
-            break;
-        const bool masked = a.mask && a.mask[e] != 0.f;
-        keys[e] = masked ? kMaskedKey : descending_key(candidate_score(a.logits[e], inverse));
-        tokens[e] = (uint32_t) e;
+    return exp(candidate_score(logit, inverse) - top);
+}
+
+// The bin of a score `distance` = top - score below the largest: 64 a unit up
+// to 16, then 64 an octave (the top bits of the distance as a float), the last
+// one for all that lie past 2^20.  Never decreasing in the distance.  A
+// NaN: before every number with the sign clear, after with it set, as the
+// ranking key has it (an infinity's distance to itself is a NaN of clear sign).
+__device__ inline int distance_bin(float logit, double inverse, double top)
+{
+    const double distance = top - candidate_score(logit, inverse);
+    if (!(distance >= 0.0))
+        return logit != logit && (__float_as_uint(logit) >> 31) ? kBins - 1 : 0;
+    if (distance < 16.0)
+        return (int) (distance * 64.0);
+    const float f = (float) fmin(distance, 1e30);
+    const int octaves = (int) (__float_as_uint(f) >> 17) - (int) (__float_as_uint(16.f) >> 17);
+    return min(kBins / 2 + octaves, kBins - 1);
+}
+
+__device__ inline void split_mass(double w, uint64_t &hi, uint64_t &lo)
+{
+    const double scaled = w * 4294967296.0;
+    const double whole = floor(scaled);
+    hi = (uint64_t) whole;
+    lo = (uint64_t) rint((scaled - whole) * 4294967296.0);
+}
+
+__device__ inline double joined_mass(uint64_t hi, uint64_t lo)
+{
+    return (double) hi * 0x1p-32 + (double) lo * 0x1p-64;
+}
+
+struct ScanShared {
+    double mass[kSampleWaves];
+    uint32_t count[kSampleWaves];
+};
+
+// Exclusive prefixes of every thread's (count, mass) over the workgroup, and
+// their totals; the order of the sums is fixed.
+__device__ inline void workgroup_scan(uint32_t count, double mass, uint32_t &countBefore,
+                                      double &massBefore, uint32_t &countTotal, double &massTotal,
+                                      ScanShared &sh)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t c = count;
+    double m = mass;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t pc = __shfl_up(c, d);
+        const double pm = __shfl_up(m, d);
+        if (lane >= d) {
+            c += pc;
+            m = pm + m;
+        }
     }
-}
-
-__global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const uint64_t *keys, int n,
-                                                                  int shift, int *hist, int tiles)
-{
-    __shared__ int counts[256];
-    counts[threadIdx.x] = 0;
-    __syncthreads();
-    for (int r = 0; r < kSortRounds; ++r) {
-        const int e = blockIdx.x * kSortTile + r * kSortThreads + threadIdx.x;
-        if (e < n)
-            atomicAdd(&counts[(keys[e] >> shift) & 255], 1);
+    __syncthreads(); // the previous scan's totals have been read
+    if (lane == 63) {
+        sh.count[wave] = c;
+        sh.mass[wave] = m;
     }
     __syncthreads();
-    hist[threadIdx.x * tiles + blockIdx.x] = counts[threadIdx.x];
+    uint32_t cb = 0, ct = 0;
+    double mb = 0.0, mt = 0.0;
+#pragma unroll
+    for (int w = 0; w < kSampleWaves; ++w) {
+        if (w == wave) {
+            cb = ct;
+            mb = mt;
+        }
+        ct += sh.count[w];
+        mt += sh.mass[w];
+    }
+    const uint32_t pc = __shfl_up(c, 1);
+    const double pm = __shfl_up(m, 1);
+    countBefore = cb + (lane > 0 ? pc : 0u);
+    massBefore = lane > 0 ? mb + pm : mb;
+    countTotal = ct;
+    massTotal = mt;
 }
 
-// Exclusive scan of the digit-major histogram: offset of (digit, tile).
-__global__ __launch_bounds__(kDrawThreads) void radix_scan_kernel(int *hist, int total)
+// A place in the ranking: the candidate of rank `rank`, or the first whose
+// running mass reaches (kReaches) or passes (kPasses) `mass`.
+enum PlaceKind { kRank, kReaches, kPasses };
+struct Place {
+    PlaceKind kind;
+    uint32_t rank;
+    double mass;
+    __device__ bool here(uint32_t countThrough, double massThrough) const
+    {
+        return kind == kRank ? countThrough > rank
+                             : (kind == kReaches ? massThrough >= mass : massThrough > mass);
+    }
+};
+
+// Candidates before a set and in it.
+struct Span {
+    uint32_t before, count;
+    double massBefore, mass;
+    int bin;
+};
+
+struct BinShared {
+    uint32_t counts[kBins];
+    double masses[kBins];
+    ScanShared scan;
+    int first, last;
+    Span span;
+};
+
+// The first bin of sh.counts / sh.masses (behind `before` candidates of
+// `massBefore`) that holds the place; the last that holds anything where none
+// does (the place lies within the sums' rounding of the end).
+__device__ inline Span find_bin(BinShared &sh, const Place &place, uint32_t before, double massBefore)
 {
-    __shared__ int sums[kDrawThreads];
     const int t = threadIdx.x;
-    const int chunk = (total + kDrawThreads - 1) / kDrawThreads;
-    const int b = min(t * chunk, total), e = min(b + chunk, total);
-    int s = 0;
-    for (int i = b; i < e; ++i)
-        s += hist[i];
-    sums[t] = s;
-    __syncthreads();
+    const uint32_t c0 = sh.counts[2 * t], c1 = sh.counts[2 * t + 1];
+    const double m0 = sh.masses[2 * t], m1 = sh.masses[2 * t + 1];
+    uint32_t cb, ct;
+    double mb, mt;
+    workgroup_scan(c0 + c1, m0 + m1, cb, mb, ct, mt, sh.scan);
+    cb += before;
+    mb += massBefore;
     if (t == 0) {
-        int running = 0;
-        for (int i = 0; i < kDrawThreads; ++i) {
-            const int v = sums[i];
-            sums[i] = running;
-            running += v;
-        }
+        sh.first = INT_MAX;
+        sh.last = 0;
     }
     __syncthreads();
-    int running = sums[t];
-    for (int i = b; i < e; ++i) {
-        const int v = hist[i];
-        hist[i] = running;
-        running += v;
-    }
+    if (c0 && place.here(cb + c0, mb + m0))
+        atomicMin(&sh.first, 2 * t);
+    else if (c1 && place.here(cb + c0 + c1, mb + m0 + m1))
+        atomicMin(&sh.first, 2 * t + 1);
+    if (c0 | c1)
+        atomicMax(&sh.last, c1 ? 2 * t + 1 : 2 * t);
+    __syncthreads();
+    const int bin = sh.first == INT_MAX ? sh.last : sh.first;
+    if (bin >> 1 == t)
+        sh.span = bin & 1 ? Span{cb + c0, c1, mb + m0, m1, bin} : Span{cb, c0, mb, m0, bin};
+    __syncthreads();
+    const Span s = sh.span;
+    __syncthreads(); // sh is rewritten by the next search
+    return s;
 }
 
-// Stable scatter: an element's place is its digit's offset for the tile,
-// plus the digit's count in earlier rounds of the tile, earlier waves of the
-// round, and earlier lanes of the wave (ballots over the digit's bits).
-__global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
-    const uint64_t *keysIn, const uint32_t *tokensIn, uint64_t *keysOut, uint32_t *tokensOut, int n,
-    int shift, const int *offsets, int tiles)
+struct RankShared {
+    uint64_t keys[kRankCap], sorted[kRankCap];
+    double masses[kRankCap];
+    ScanShared scan;
+    uint64_t low, high;
+    uint32_t found, gathered;
+    uint32_t rank;
+    double mass;
+    uint32_t token;
+};
+
+struct Candidate {
+    uint32_t rank, token;
+    double massThrough;
+};
+
+// The place's candidate among those of `span` (contiguous in `keys`).
+__device__ inline Candidate locate(const uint64_t *keys, Span span, const Place &place,
+                                   double inverse, double top, BinShared &bs, RankShared &rs)
 {
-    constexpr int kWaves = kSortThreads / 64;
-    __shared__ int running[256], base[256];
-    __shared__ int waveCount[kWaves][256], wavePrefix[kWaves][256];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    running[t] = 0;
-    const uint64_t below = (1ull << lane) - 1;
-    for (int r = 0; r < kSortRounds; ++r) {
-        const int e = blockIdx.x * kSortTile + r * kSortThreads + t;
-        const bool valid = e < n;
-        const uint64_t key = valid ? keysIn[e] : 0;
-        const uint32_t token = valid ? tokensIn[e] : 0;
-        const int d = (int) ((key >> shift) & 255);
-        uint64_t peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const uint64_t m = __ballot((d >> b) & 1);
-            peers &= ((d >> b) & 1) ? m : ~m;
+    const int t = threadIdx.x;
+    const uint32_t size = span.count; // of `keys`
+    uint64_t low = 0, high = ~0ull;   // the set: keys in [low, high]
+    while (span.count > (uint32_t) kRankCap) {
+        // the range the set's keys cover, in 2048 bins of a power of two
+        if (t == 0) {
+            rs.low = ~0ull;
+            rs.high = 0ull;
         }
-        const int rank = __popcll(peers & below);
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w)
-            waveCount[w][t] = 0;
+        for (int b = t; b < kBins; b += kSampleThreads)
+            bs.counts[b] = 0u;
         __syncthreads();
-        if (valid && (peers >> lane) == 1ull) // the last lane of its digit's peers
-            waveCount[wave][d] = __popcll(peers);
-        __syncthreads();
-        {
-            int s = 0;
-#pragma unroll
-            for (int w = 0; w < kWaves; ++w) {
-                wavePrefix[w][t] = s;
-                s += waveCount[w][t];
+        uint64_t lo = ~0ull, hi = 0ull;
+        for (uint32_t i = t; i < size; i += kSampleThreads) {
+            const uint64_t k = keys[i];
+            if (k >= low && k <= high) {
+                lo = k < lo ? k : lo;
+                hi = k > hi ? k : hi;
             }
-            base[t] = running[t];
-            running[t] += s;
         }
+        atomicMin((unsigned long long *) &rs.low, (unsigned long long) lo);
+        atomicMax((unsigned long long *) &rs.high, (unsigned long long) hi);
         __syncthreads();
-        if (valid) {
-            const int at = offsets[d * tiles + blockIdx.x] + base[d] + wavePrefix[wave][d] + rank;
-            keysOut[at] = key;
-            tokensOut[at] = token;
+        low = rs.low;
+        high = rs.high;
+        int shift = 0;
+        while (((high - low) >> shift) >= (uint64_t) kBins)
+            ++shift;
+        // a candidate's mass as integers, so the sums' order does not matter:
+        // the high part in masses, the low part below 2^-32 a second time round
+        uint64_t *parts = reinterpret_cast<uint64_t *>(bs.masses);
+        double total[2];
+        for (int part = 0; part < 2; ++part) {
+            for (int b = t; b < kBins; b += kSampleThreads)
+                parts[b] = 0ull;
+            __syncthreads();
+            for (uint32_t i = t; i < size; i += kSampleThreads) {
+                const uint64_t k = keys[i];
+                if (k < low || k > high)
+                    continue;
+                const int b = (int) ((k - low) >> shift);
+                uint64_t mh, ml;
+                split_mass(candidate_weight(logit_of_key(k), inverse, top), mh, ml);
+                atomicAdd((unsigned long long *) &parts[b], (unsigned long long) (part ? ml : mh));
+                if (part == 0)
+                    atomicAdd(&bs.counts[b], 1u);
+            }
+            __syncthreads();
+            if (part == 0) {
+                total[0] = (double) parts[2 * t] * 0x1p-32;
+                total[1] = (double) parts[2 * t + 1] * 0x1p-32;
+            } else {
+                total[0] += (double) parts[2 * t] * 0x1p-64;
+                total[1] += (double) parts[2 * t + 1] * 0x1p-64;
+            }
+            __syncthreads();
         }
+        bs.masses[2 * t] = total[0];
+        bs.masses[2 * t + 1] = total[1];
         __syncthreads();
+        span = find_bin(bs, place, span.before, span.massBefore);
+        low += (uint64_t) span.bin << shift;
+        const uint64_t end = low + ((1ull << shift) - 1);
+        high = end < high ? end : high;
     }
-}
-
-// The first i in [0, count) (in order) whose running sum of value(i) makes
-// crosses(sum) true, or -1.  Each thread sums a contiguous chunk, the chunk
-// sums are scanned in order, and each thread then walks its own chunk from
-// its prefix; the smallest index found wins.  crosses is monotone and the
-// values are not negative, so this is the sequential walk up to the rounding
-// of the sums.  All threads of the workgroup call it.
-template <typename Value, typename Crosses>
-__device__ int first_crossing(int count, Value value, Crosses crosses, double *sums, int *first)
-{
-    const int t = threadIdx.x;
-    const int chunk = (count + kDrawThreads - 1) / kDrawThreads;
-    const int b = min(t * chunk, count), e = min(b + chunk, count);
-    double s = 0.0;
-    for (int i = b; i < e; ++i)
-        s += value(i);
-    sums[t] = s;
-    if (t == 0)
-        *first = INT_MAX;
-    __syncthreads();
+    // few enough: each thread's candidate takes its place among the others
     if (t == 0) {
-        double running = 0.0;
-        for (int i = 0; i < kDrawThreads; ++i) {
-            const double v = sums[i];
-            sums[i] = running;
-            running += v;
-        }
+        rs.gathered = 0u;
+        rs.found = UINT_MAX;
     }
     __syncthreads();
-    double m = sums[t];
-    for (int i = b; i < e; ++i) {
-        const double v = value(i);
-        m += v;
-        if (v > 0.0 && crosses(m)) { // a zero term never makes the first crossing
-            atomicMin(first, i);
-            break;
-        }
+    for (uint32_t i = t; i < size; i += kSampleThreads) {
+        const uint64_t k = keys[i];
+        if (k >= low && k <= high)
+            rs.keys[atomicAdd(&rs.gathered, 1u)] = k;
     }
     __syncthreads();
-    const int found = *first;
-    __syncthreads(); // sums and first are reused by the next call
-    return found == INT_MAX ? -1 : found;
+    const uint32_t n = span.count;
+    if (t < (int) n) {
+        const uint64_t mine = rs.keys[t];
+        uint32_t rank = 0;
+        for (uint32_t i = 0; i < n; ++i)
+            rank += rs.keys[i] < mine ? 1u : 0u;
+        rs.sorted[rank] = mine;
+    }
+    __syncthreads();
+    double weight = 0.0;
+    if (t < (int) n)
+        weight = candidate_weight(logit_of_key(rs.sorted[t]), inverse, top);
+    uint32_t cb, ct;
+    double mb, mt;
+    workgroup_scan(t < (int) n ? 1u : 0u, weight, cb, mb, ct, mt, rs.scan);
+    const uint32_t through = span.before + cb + 1;
+    const double massThrough = span.massBefore + (mb + weight);
+    if (t < (int) n && (place.here(through, massThrough) || t == (int) n - 1))
+        atomicMin(&rs.found, (uint32_t) t); // the last where none holds it: within rounding
+    __syncthreads();
+    if (t == (int) rs.found) {
+        rs.rank = through - 1;
+        rs.mass = massThrough;
+        rs.token = (uint32_t) rs.sorted[t];
+    }
+    __syncthreads();
+    const Candidate c{rs.rank, rs.token, rs.mass};
+    __syncthreads(); // rs is rewritten by the next search
+    return c;
 }
 
-// The sum of value(i) over [0, count): chunk sums added in chunk order, the
-// same total in every thread.
-template <typename Value>
-__device__ double ordered_total(int count, Value value, double *sums)
+// The whole row's state from its chunks' (every thread takes part).
+__device__ inline ChunkState row_state(const ChunkState *chunks, int count)
 {
+    __shared__ double sLargest[kSampleWaves];
+    __shared__ int sCount, sLast, sBad;
     const int t = threadIdx.x;
-    const int chunk = (count + kDrawThreads - 1) / kDrawThreads;
-    const int b = min(t * chunk, count), e = min(b + chunk, count);
-    double s = 0.0;
-    for (int i = b; i < e; ++i)
-        s += value(i);
-    sums[t] = s;
-    __syncthreads();
-    double total = 0.0;
-    for (int i = 0; i < kDrawThreads; ++i)
-        total += sums[i];
-    __syncthreads();
-    return total;
-}
-
-// Sampler::sample after the scores (Sampler.cpp:101-205).  `ranked`: the keys
-// and tokens hold the row sorted by rank (masked tokens last).
-__global__ __launch_bounds__(kDrawThreads) void sample_draw_kernel(SampleArgs a, const uint64_t *keys,
-                                                                   const uint32_t *tokens, int ranked)
-{
-    __shared__ double sums[kDrawThreads];
-    __shared__ double sLargest;
-    __shared__ int sCount, sFirst, sLast;
-    const int t = threadIdx.x, V = a.vocab;
-    const double u = a.draws[min(*a.draw_index, a.draw_count - 1)];
-    const double inverse = 1.0 / (double) a.temperature;
-    auto masked = [&](int i) { return a.mask && a.mask[i] != 0.f; };
-
     if (t == 0) {
         sCount = 0;
         sLast = -1;
+        sBad = 0;
     }
     __syncthreads();
     double largest = -DBL_MAX;
-    int count = 0, last = -1;
-    for (int i = t; i < V; i += kDrawThreads)
-        if (!masked(i)) {
-            largest = fmax(largest, candidate_score(a.logits[i], inverse));
-            ++count;
-            last = i;
-        }
+    for (int i = t; i < count; i += kSampleThreads) {
+        const ChunkState c = chunks[i];
+        largest = fmax(largest, c.largest);
+        atomicAdd(&sCount, c.count);
+        atomicMax(&sLast, c.last);
+        if (c.bad)
+            atomicOr(&sBad, 1);
+    }
     largest = wave_max_d(largest);
     if ((t & 63) == 0)
-        sums[t >> 6] = largest;
-    atomicAdd(&sCount, count);
-    atomicMax(&sLast, last);
+        sLargest[t >> 6] = largest;
+    __syncthreads();
+    ChunkState s{};
+    s.largest = -DBL_MAX;
+    for (int w = 0; w < kSampleWaves; ++w)
+        s.largest = fmax(s.largest, sLargest[w]);
+    s.count = sCount;
+    s.last = sLast;
+    s.bad = sBad;
+    return s;
+}
+
+__device__ inline bool masked(const SampleArgs &a, int token)
+{
+    return a.mask && a.mask[token] != 0.f;
+}
+
+__global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a, SampleWorkspace w)
+{
+    __shared__ double sLargest[kSampleWaves];
+    __shared__ int sCount, sLast, sBad;
+    const int t = threadIdx.x;
+    for (int b = blockIdx.x * kSampleThreads + t; b < kBins; b += gridDim.x * kSampleThreads) {
+        w.counts[b] = 0u;
+        w.cursors[b] = 0u;
+        w.massHi[b] = 0ull;
+        w.massLo[b] = 0ull;
+    }
+    if (t == 0) {
+        sCount = 0;
+        sLast = -1;
+        sBad = 0;
+    }
+    __syncthreads();
+    const double inverse = 1.0 / (double) a.temperature;
+    const int64_t first = (int64_t) blockIdx.x * kChunkTokens + t;
+    float logit[kChunkRounds];
+    bool live[kChunkRounds];
+#pragma unroll
+    for (int r = 0; r < kChunkRounds; ++r) {
+        const int64_t e = first + r * kSampleThreads;
+        live[r] = e < a.vocab && !masked(a, (int) e);
+        logit[r] = a.logits[e < a.vocab ? e : 0];
+    }
+    double largest = -DBL_MAX;
+    int count = 0, last = -1, bad = 0;
+#pragma unroll
+    for (int r = 0; r < kChunkRounds; ++r)
+        if (live[r]) {
+            largest = fmax(largest, candidate_score(logit[r], inverse));
+            ++count;
+            last = (int) (first + r * kSampleThreads);
+            bad |= !(logit[r] < INFINITY);
+        }
+    largest = wave_max_d(largest);
+    const double deepest = wave_max_d((double) last); // exact: below 2^31
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1)
+        count += __shfl_xor(count, d);
+    const bool anyBad = __any(bad) != 0;
+    if ((t & 63) == 0) { // one atomic a wave
+        sLargest[t >> 6] = largest;
+        atomicAdd(&sCount, count);
+        atomicMax(&sLast, (int) deepest);
+        if (anyBad)
+            atomicOr(&sBad, 1);
+    }
     __syncthreads();
     if (t == 0) {
         double m = -DBL_MAX;
-        for (int w = 0; w < kDrawThreads / 64; ++w)
-            m = fmax(m, sums[w]);
-        sLargest = m;
+        for (int i = 0; i < kSampleWaves; ++i)
+            m = fmax(m, sLargest[i]);
+        w.chunks[blockIdx.x] = ChunkState{m, 0.0, sCount, sLast, sBad, 0};
+    }
+}
+
+__global__ __launch_bounds__(kSampleThreads) void sample_bins_kernel(SampleArgs a, SampleWorkspace w,
+                                                                     int ranked)
+{
+    __shared__ uint32_t sCounts[kBins];
+    __shared__ unsigned long long sHi[kBins], sLo[kBins];
+    __shared__ ScanShared sScan;
+    const int t = threadIdx.x;
+    const int64_t first = (int64_t) blockIdx.x * kChunkTokens + t;
+    float logit[kChunkRounds];
+    bool live[kChunkRounds];
+#pragma unroll
+    for (int r = 0; r < kChunkRounds; ++r) {
+        const int64_t e = first + r * kSampleThreads;
+        live[r] = e < a.vocab && !masked(a, (int) e);
+        logit[r] = a.logits[e < a.vocab ? e : 0];
+    }
+    if (ranked)
+        for (int b = t; b < kBins; b += kSampleThreads) {
+            sCounts[b] = 0u;
+            sHi[b] = 0ull;
+            sLo[b] = 0ull;
+        }
+    const ChunkState row = row_state(w.chunks, w.chunkCount); // (syncs)
+    const double inverse = 1.0 / (double) a.temperature, top = row.largest;
+    double mass = 0.0;
+#pragma unroll
+    for (int r = 0; r < kChunkRounds; ++r) {
+        if (!live[r])
+            continue;
+        const double weight = candidate_weight(logit[r], inverse, top);
+        mass += weight;
+        if (ranked) {
+            const int b = distance_bin(logit[r], inverse, top);
+            uint64_t hi = 0, lo = 0;
+            if (!row.bad) // else no mass is a number, and none is used
+                split_mass(weight, hi, lo);
+            atomicAdd(&sCounts[b], 1u);
+            if (hi)
+                atomicAdd(&sHi[b], (unsigned long long) hi);
+            if (lo)
+                atomicAdd(&sLo[b], (unsigned long long) lo);
+        }
+    }
+    uint32_t cb, ct;
+    double mb, mt;
+    workgroup_scan(0u, mass, cb, mb, ct, mt, sScan); // (syncs)
+    if (t == 0) {
+        w.chunks[blockIdx.x].mass = mt;
+        if (blockIdx.x == 0)
+            *w.row = row;
+    }
+    if (ranked)
+        for (int b = t; b < kBins; b += kSampleThreads)
+            if (sCounts[b]) {
+                atomicAdd(&w.counts[b], sCounts[b]);
+                atomicAdd((unsigned long long *) &w.massHi[b], sHi[b]);
+                atomicAdd((unsigned long long *) &w.massLo[b], sLo[b]);
+            }
+}
+
+__device__ inline void load_bins(const SampleWorkspace &w, BinShared &sh)
+{
+    for (int b = threadIdx.x; b < kBins; b += kSampleThreads) {
+        sh.counts[b] = w.counts[b];
+        sh.masses[b] = joined_mass(w.massHi[b], w.massLo[b]);
     }
     __syncthreads();
-    const int n = sCount;
-    const double top = sLargest;
-    uint32_t chosen = 0;
-    if (n > 0 && (!ranked || !((a.top_k > 0 && a.top_k < n) || a.top_p < 1.f))) {
-        // no cut: every unmasked token in token order
-        auto weight = [&](int i) -> double {
-            return masked(i) ? 0.0 : exp(candidate_score(a.logits[i], inverse) - top);
-        };
-        const double total = ordered_total(V, weight, sums);
-        const int at = first_crossing(
-            V, [&](int i) { return weight(i) / total; }, [&](double m) { return u < m; }, sums,
-            &sFirst);
-        chosen = (uint32_t) (at >= 0 ? at : sLast);
-    } else if (n > 0) {
-        // the ranked candidates: the top k, then the top-p prefix
-        int kept = (a.top_k > 0 && a.top_k < n) ? a.top_k : n;
-        auto weight = [&](int i) { return exp(score_of_key(keys[i]) - top); };
-        if (a.top_p < 1.f) {
-            const double total = ordered_total(kept, weight, sums);
-            const double wanted = (double) a.top_p;
-            const int at = first_crossing(
-                kept, [&](int i) { return weight(i) / total; },
-                [&](double m) { return !(m < wanted); }, sums, &sFirst);
-            kept = at >= 0 ? at + 1 : kept;
+}
+
+// Whether any cut applies to a row of n candidates, and how many the first
+// keeps.
+__device__ inline bool cut(const SampleArgs &a, int n)
+{
+    return (a.top_k > 0 && a.top_k < n) || a.top_p < 1.f;
+}
+
+__device__ inline int first_kept(const SampleArgs &a, int n)
+{
+    return a.top_k > 0 && a.top_k < n ? a.top_k : n;
+}
+
+__global__ __launch_bounds__(kSampleThreads) void sample_gather_kernel(SampleArgs a, SampleWorkspace w)
+{
+    __shared__ BinShared sh;
+    __shared__ uint32_t sOffset[kBins], sMine[kBins], sBase[kBins];
+    const int t = threadIdx.x;
+    const int64_t first = (int64_t) blockIdx.x * kChunkTokens + t;
+    float logit[kChunkRounds];
+    bool live[kChunkRounds];
+#pragma unroll
+    for (int r = 0; r < kChunkRounds; ++r) {
+        const int64_t e = first + r * kSampleThreads;
+        live[r] = e < a.vocab && !masked(a, (int) e);
+        logit[r] = a.logits[e < a.vocab ? e : 0];
+    }
+    const ChunkState row = *w.row;
+    const int n = row.count;
+    if (n == 0 || !cut(a, n))
+        return;
+    const double inverse = 1.0 / (double) a.temperature, top = row.largest;
+    load_bins(w, sh);
+    // the bins' places, and the last bin that the draw reads: the k-th
+    // candidate's (whose mass the other searches need), else the one where the
+    // row's mass reaches p, else the last candidate's
+    uint32_t cb, ct;
+    double mb, mt;
+    workgroup_scan(sh.counts[2 * t] + sh.counts[2 * t + 1], sh.masses[2 * t] + sh.masses[2 * t + 1], cb,
+                   mb, ct, mt, sh.scan);
+    sOffset[2 * t] = cb;
+    sOffset[2 * t + 1] = cb + sh.counts[2 * t];
+    sMine[2 * t] = 0u;
+    sMine[2 * t + 1] = 0u;
+    const int kept = first_kept(a, n);
+    const bool byMass = kept == n && !row.bad && mt > 0.0;
+    const Place end{byMass ? kReaches : kRank, (uint32_t) kept - 1u,
+                    (double) a.top_p * mt * (1.0 + 1e-9)};
+    const int lastBin = find_bin(sh, end, 0u, 0.0).bin;
+    int bin[kChunkRounds];
+    uint32_t place[kChunkRounds];
+#pragma unroll
+    for (int r = 0; r < kChunkRounds; ++r) {
+        bin[r] = live[r] ? distance_bin(logit[r], inverse, top) : kBins;
+        if (bin[r] <= lastBin)
+            place[r] = atomicAdd(&sMine[bin[r]], 1u);
+    }
+    __syncthreads();
+    for (int b = t; b <= lastBin; b += kSampleThreads)
+        if (sMine[b])
+            sBase[b] = sOffset[b] + atomicAdd(&w.cursors[b], sMine[b]);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kChunkRounds; ++r)
+        if (bin[r] <= lastBin)
+            w.gathered[sBase[bin[r]] + place[r]] =
+                ranking_key(logit[r], (uint32_t) (first + r * kSampleThreads));
+}
+
+// The first token, in token order, whose running mass passes `target` (the
+// chunks' masses, then the chunk's own weights); -1 where none does.
+__device__ inline int token_order_draw(const SampleArgs &a, const SampleWorkspace &w, double uniform,
+                                       double inverse, double top, ScanShared &scan)
+{
+    __shared__ int sFirst;
+    __shared__ double sBefore;
+    const int t = threadIdx.x;
+    const int per = (w.chunkCount + kSampleThreads - 1) / kSampleThreads;
+    const int c0 = min(t * per, w.chunkCount), c1 = min(c0 + per, w.chunkCount);
+    double mass = 0.0;
+    for (int i = c0; i < c1; ++i)
+        mass += w.chunks[i].mass;
+    uint32_t cb, ct;
+    double before, total;
+    workgroup_scan(0u, mass, cb, before, ct, total, scan);
+    if (t == 0)
+        sFirst = INT_MAX;
+    __syncthreads();
+    const double target = uniform * total;
+    double through = before;
+    for (int i = c0; i < c1; ++i) {
+        through += w.chunks[i].mass;
+        if (through > target) {
+            atomicMin(&sFirst, i);
+            break;
         }
-        const double total = ordered_total(kept, weight, sums);
-        const int at = first_crossing(
-            kept, [&](int i) { return weight(i) / total; }, [&](double m) { return u < m; }, sums,
-            &sFirst);
-        chosen = tokens[at >= 0 ? at : kept - 1];
+    }
+    __syncthreads();
+    const int chunk = sFirst;
+    __syncthreads();
+    if (chunk == INT_MAX)
+        return -1;
+    if (chunk >= c0 && chunk < c1) {
+        double b = before;
+        for (int i = c0; i < chunk; ++i)
+            b += w.chunks[i].mass;
+        sBefore = b;
+    }
+    if (t == 0)
+        sFirst = INT_MAX;
+    __syncthreads();
+    // kChunkRounds consecutive tokens a thread
+    double weight[kChunkRounds], sum = 0.0;
+    int last = -1;
+    const int64_t first = (int64_t) chunk * kChunkTokens + t * kChunkRounds;
+#pragma unroll
+    for (int r = 0; r < kChunkRounds; ++r) {
+        const int64_t e = first + r;
+        const bool live = e < a.vocab && !masked(a, (int) e);
+        weight[r] = live ? candidate_weight(a.logits[e], inverse, top) : 0.0;
+        sum += weight[r];
+        last = weight[r] > 0.0 ? (int) e : last;
+    }
+    double mine, all;
+    workgroup_scan(0u, sum, cb, mine, ct, all, scan);
+    __shared__ int sLast;
+    if (t == 0)
+        sLast = -1;
+    __syncthreads();
+    atomicMax(&sLast, last);
+    double running = sBefore + mine;
+#pragma unroll
+    for (int r = 0; r < kChunkRounds; ++r) {
+        running += weight[r];
+        if (weight[r] > 0.0 && running > target) {
+            atomicMin(&sFirst, (int) (first + r));
+            break;
+        }
+    }
+    __syncthreads();
+    // the chunk's sum in this order may round below the target it passed
+    return sFirst == INT_MAX ? sLast : sFirst;
+}
+
+__global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(SampleArgs a, SampleWorkspace w)
+{
+    __shared__ BinShared bins;
+    __shared__ RankShared ranks;
+    const int t = threadIdx.x;
+    const double uniform = a.draws ? a.draws[min(*a.draw_index, a.draw_count - 1)] : a.uniform;
+    const ChunkState row = *w.row;
+    const double inverse = 1.0 / (double) a.temperature, top = row.largest;
+    const int n = row.count;
+    uint32_t chosen = 0;
+    if (n > 0 && !cut(a, n)) {
+        const int at = row.bad ? -1 : token_order_draw(a, w, uniform, inverse, top, bins.scan);
+        chosen = (uint32_t) (at >= 0 ? at : row.last);
+    } else if (n > 0) {
+        load_bins(w, bins);
+        uint32_t cb, ct;
+        double mb, all;
+        workgroup_scan(0u, bins.masses[2 * t] + bins.masses[2 * t + 1], cb, mb, ct, all, bins.scan);
+        // the bin of a place, and the candidate in it (its bin's gathered
+        // candidates; `locate` may use the bins' space, which is then loaded
+        // again)
+        auto find = [&](const Place &place) {
+            const Span span = find_bin(bins, place, 0u, 0.0);
+            const Candidate c = locate(w.gathered + span.before, span, place, inverse, top, bins, ranks);
+            if (span.count > (uint32_t) kRankCap)
+                load_bins(w, bins);
+            return c;
+        };
+        const bool sums = !row.bad && all > 0.0; // else no running mass is a number
+        int kept = first_kept(a, n);
+        double mass = all;
+        Candidate end{};
+        bool known = false; // `end` is the last kept candidate
+        if (kept < n) {
+            end = find(Place{kRank, (uint32_t) kept - 1u, 0.0});
+            known = true;
+            mass = end.massThrough;
+        }
+        if (sums && a.top_p < 1.f) {
+            const Candidate c = find(Place{kReaches, 0u, (double) a.top_p * mass});
+            if ((int) c.rank < kept - 1 || !known) {
+                end = c;
+                known = true;
+                kept = (int) c.rank + 1;
+                mass = c.massThrough;
+            }
+        }
+        bool drawn = false;
+        if (sums) {
+            const Candidate c = find(Place{kPasses, 0u, uniform * mass});
+            drawn = (int) c.rank < kept;
+            chosen = c.token;
+        }
+        if (!drawn) {
+            if (!known)
+                end = find(Place{kRank, (uint32_t) kept - 1u, 0.0});
+            chosen = end.token;
+        }
     }
     if (t == 0) {
         if (a.sequence)
             a.sequence[*a.position + a.offset] = chosen;
         if (a.token_out)
             *a.token_out = chosen;
-        *a.draw_index += 1;
+        if (a.draws)
+            *a.draw_index += 1;
     }
 }
 
 SampleWorkspace carve(void *workspace, int vocab)
 {
     SampleWorkspace w{};
-    w.tiles = sort_tiles(vocab);
-    uint8_t *p = static_cast<uint8_t *>(workspace);
-    for (int i = 0; i < 2; ++i) {
-        w.keys[i] = reinterpret_cast<uint64_t *>(p);
-        p += align256((size_t) vocab * 8);
-        w.tokens[i] = reinterpret_cast<uint32_t *>(p);
-        p += align256((size_t) vocab * 4);
-    }
-    w.hist = reinterpret_cast<int *>(p);
+    w.chunkCount = sample_chunks(vocab);
+    uint8_t *p = reinterpret_cast<uint8_t *>(align256(reinterpret_cast<uintptr_t>(workspace)));
+    auto take = [&](size_t bytes) {
+        uint8_t *at = p;
+        p += align256(bytes);
+        return at;
+    };
+    w.row = reinterpret_cast<ChunkState *>(take(sizeof(ChunkState)));
+    w.chunks = reinterpret_cast<ChunkState *>(take(w.chunkCount * sizeof(ChunkState)));
+    w.counts = reinterpret_cast<uint32_t *>(take(kBins * sizeof(uint32_t)));
+    w.cursors = reinterpret_cast<uint32_t *>(take(kBins * sizeof(uint32_t)));
+    w.massHi = reinterpret_cast<uint64_t *>(take(kBins * sizeof(uint64_t)));
+    w.massLo = reinterpret_cast<uint64_t *>(take(kBins * sizeof(uint64_t)));
+    w.gathered = reinterpret_cast<uint64_t *>(p);
     return w;
 }
 
@@ -345,8 +784,9 @@ size_t sample_workspace_bytes(int vocab)
 {
     if (vocab <= 0)
         return 0;
-    return 2 * (align256((size_t) vocab * 8) + align256((size_t) vocab * 4))
-           + align256((size_t) 256 * sort_tiles(vocab) * 4);
+    return align256(sizeof(ChunkState)) + align256(sample_chunks(vocab) * sizeof(ChunkState))
+           + 2 * align256(kBins * sizeof(uint32_t)) + 2 * align256(kBins * sizeof(uint64_t))
+           + align256((size_t) vocab * sizeof(uint64_t)) + 256; // and its alignment
 }
 
 bool sampling_options_valid(float temperature, int top_k, float top_p)
@@ -358,7 +798,7 @@ bool sampling_options_valid(float temperature, int top_k, float top_p)
 hipError_t launch_sample(const SampleArgs &a, void *workspace, size_t workspace_bytes,
                          hipStream_t stream)
 {
-    if (!a.logits || a.vocab <= 0 || !a.draws || a.draw_count <= 0 || !a.draw_index
+    if (!a.logits || a.vocab <= 0 || (a.draws && (a.draw_count <= 0 || !a.draw_index))
         || !(a.temperature > 0.f)
         || !sampling_options_valid(a.temperature, a.top_k, a.top_p)
         || (!a.sequence && !a.token_out) || (a.sequence && !a.position) || !workspace
@@ -366,23 +806,12 @@ hipError_t launch_sample(const SampleArgs &a, void *workspace, size_t workspace_
         return hipErrorInvalidValue;
     const SampleWorkspace w = carve(workspace, a.vocab);
     const bool ranked = a.top_k > 0 || a.top_p < 1.f;
-    if (ranked) {
-        hipLaunchKernelGGL(sample_keys_kernel, dim3(w.tiles), dim3(kSortThreads), 0, stream, a,
-                           w.keys[0], w.tokens[0]);
-        for (int pass = 0; pass < 8; ++pass) {
-            const int in = pass & 1, shift = 8 * pass;
-            hipLaunchKernelGGL(radix_hist_kernel, dim3(w.tiles), dim3(kSortThreads), 0, stream,
-                               w.keys[in], a.vocab, shift, w.hist, w.tiles);
-            hipLaunchKernelGGL(radix_scan_kernel, dim3(1), dim3(kDrawThreads), 0, stream, w.hist,
-                               256 * w.tiles);
-            hipLaunchKernelGGL(radix_scatter_kernel, dim3(w.tiles), dim3(kSortThreads), 0, stream,
-                               w.keys[in], w.tokens[in], w.keys[in ^ 1], w.tokens[in ^ 1], a.vocab,
-                               shift, w.hist, w.tiles);
-        }
-    }
-    // eight passes leave the ranked row back in buffer 0
-    hipLaunchKernelGGL(sample_draw_kernel, dim3(1), dim3(kDrawThreads), 0, stream, a, w.keys[0],
-                       w.tokens[0], ranked ? 1 : 0);
+    const dim3 grid(w.chunkCount), block(kSampleThreads);
+    hipLaunchKernelGGL(sample_max_kernel, grid, block, 0, stream, a, w);
+    hipLaunchKernelGGL(sample_bins_kernel, grid, block, 0, stream, a, w, ranked ? 1 : 0);
+    if (ranked)
+        hipLaunchKernelGGL(sample_gather_kernel, grid, block, 0, stream, a, w);
+    hipLaunchKernelGGL(sample_draw_kernel, dim3(1), block, 0, stream, a, w);
     return hipGetLastError();
 }
 

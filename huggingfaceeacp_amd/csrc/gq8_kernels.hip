@@ -67,6 +67,57 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_kernel(const float *__
     quantize_in_group(x[i], threadIdx.x & 31, q + i, scales + i / kBlock);
 }
 
+// Eight elements a thread: the byte and scale arithmetic of the block's four
+// threads is done once each instead of once an element, and values and bytes
+// move 32 and 8 bytes at a time.  The same maxima, scales and bytes as
+// quantize_in_group.  The four lanes of a block are active together.
+__device__ inline void quantize_eight(const float (&v)[8], uint8_t *q, uint16_t *scaleSlot)
+{
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        amax = fmaxf(amax, fabsf(v[i]));
+    amax = fmaxf(amax, __shfl_xor(amax, 1));
+    amax = fmaxf(amax, __shfl_xor(amax, 2));
+    const uint16_t bits = scale_bits_from_amax(amax);
+    const float scale = half_value(bits);
+    const float inverse = quantize_hint(scale);
+    uint32_t packed[2] = {0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        packed[i / 4] |= (uint32_t) (uint8_t) (int8_t) quantize_in_block(v[i], bits, scale, inverse)
+                         << (8 * (i % 4));
+    *reinterpret_cast<uint2 *>(q) = make_uint2(packed[0], packed[1]);
+    if ((threadIdx.x & 3) == 0)
+        *scaleSlot = bits;
+}
+
+__device__ inline void load_eight(const float *p, float (&v)[8])
+{
+    const float4 a = reinterpret_cast<const float4 *>(p)[0], b = reinterpret_cast<const float4 *>(p)[1];
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+
+__device__ inline void store_eight(float *p, const float (&v)[8])
+{
+    reinterpret_cast<float4 *>(p)[0] = float4{v[0], v[1], v[2], v[3]};
+    reinterpret_cast<float4 *>(p)[1] = float4{v[4], v[5], v[6], v[7]};
+}
+
+__global__ __launch_bounds__(kThreads) void quantize_rows_wide_kernel(const float *__restrict__ x,
+                                                                      int64_t elements,
+                                                                      uint8_t *__restrict__ q,
+                                                                      uint16_t *__restrict__ scales)
+{
+    const int64_t i = 8 * ((int64_t) blockIdx.x * kThreads + threadIdx.x);
+    if (i >= elements) // whole blocks: their four threads leave together
+        return;
+    float v[8];
+    load_eight(x + i, v);
+    quantize_eight(v, q + i, scales + i / kBlock);
+}
+
 // ---- embedding gather (Embed.h:45-82) ------------------------------------
 // Row r embeds tokens[*pos_ptr + r] (one sequence), or with row_positions
 // tokens[r * slot_stride + row_positions[r]] (row r of a lockstep batch, each
@@ -104,6 +155,36 @@ __global__ __launch_bounds__(kThreads) void embed_kernel(const uint32_t *__restr
     const uint16_t bits = reinterpret_cast<const uint16_t *>(table + elements)[e / kBlock];
     const float gathered = half_value(bits) * (float) (int8_t) table[e];
     out[(int64_t) row * width + c] = (float) ((double) scale * (double) gathered);
+}
+
+// Rows of tokens[*pos_ptr + row], eight channels a thread (embed_kernel's
+// values).
+__global__ __launch_bounds__(kThreads) void embed_wide_kernel(const uint32_t *__restrict__ tokens,
+                                                              const int *pos_ptr,
+                                                              const uint8_t *__restrict__ table,
+                                                              int64_t vocab, int width, float scale,
+                                                              float *__restrict__ out, int64_t pieces)
+{
+    const int64_t i = (int64_t) blockIdx.x * kThreads + threadIdx.x;
+    if (i >= pieces)
+        return;
+    const int perRow = width / 8;
+    const int64_t row = i / perRow;
+    const int c = (int) (i % perRow) * 8;
+    uint32_t token = tokens[(int64_t) (pos_ptr ? *pos_ptr : 0) + row];
+    if (token >= (uint32_t) vocab) // ids are validated on the host; a guard, not a rule
+        token = 0;
+    const int64_t e = (int64_t) token * width + c;
+    const uint16_t bits = reinterpret_cast<const uint16_t *>(table + vocab * width)[e / kBlock];
+    const float blockScale = half_value(bits);
+    const uint2 bytes = *reinterpret_cast<const uint2 *>(table + e);
+    float v[8];
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        const int8_t stored = (int8_t) ((b < 4 ? bytes.x : bytes.y) >> (8 * (b % 4)));
+        v[b] = (float) ((double) scale * (double) (blockScale * (float) stored));
+    }
+    store_eight(out + row * width + c, v);
 }
 
 // ---- RMSNorm, optionally fused with the activation quantization ---------
@@ -821,6 +902,33 @@ __global__ __launch_bounds__(kThreads) void geglu_kernel(const float *__restrict
                               + at / kBlock);
 }
 
+// Eight outputs a thread (geglu_kernel's values and bytes): the one-output form
+// computes each block's scale 32 times over and stores a byte a lane.  2048
+// rows of 16384: 144 -> 88 us (304 MB, which the copy rate allows in 62).
+__global__ __launch_bounds__(kThreads) void geglu_wide_kernel(const float *__restrict__ fused,
+                                                              int rows, int intermediate,
+                                                              float *__restrict__ out,
+                                                              uint8_t *__restrict__ q8)
+{
+    const int row = blockIdx.y;
+    const int i = 8 * (blockIdx.x * kThreads + threadIdx.x);
+    if (i >= intermediate) // whole blocks: their four threads leave together
+        return;
+    const float *f = fused + (int64_t) row * 2 * intermediate + i;
+    float gate[8], up[8], v[8];
+    load_eight(f, gate);
+    load_eight(f + intermediate, up);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        v[k] = geglu(gate[k], up[k]);
+    const int64_t at = (int64_t) row * intermediate + i;
+    if (out)
+        store_eight(out + at, v);
+    if (q8)
+        quantize_eight(v, q8 + at,
+                       reinterpret_cast<uint16_t *>(q8 + (int64_t) rows * intermediate) + at / kBlock);
+}
+
 // ---- argmax (Argmax.h:47-200) --------------------------------------------------
 struct Candidate {
     float value;
@@ -910,6 +1018,17 @@ inline unsigned blocks_for(int64_t n, int per)
     return (unsigned) ((n + per - 1) / per);
 }
 
+bool aligned_to(const void *p, uintptr_t bytes)
+{
+    return reinterpret_cast<uintptr_t>(p) % bytes == 0;
+}
+
+// The kernels of eight values a thread take over where there are enough values
+// to fill the chip with an eighth of the threads (2048 rows of 2048: quantize
+// 9.3 -> 5.2 us, embed 9.7 -> 6.1); below, more threads with a value each end
+// sooner (geglu of one row of 16384 3.5 against 4.3 us, even at 48 rows).
+constexpr int64_t kWideElements = 1 << 20;
+
 int argmax_groups(int length)
 {
     const int per = kThreads * kArgmaxPerThread;
@@ -926,6 +1045,11 @@ hipError_t launch_quantize(const float *x, int64_t elements, uint8_t *q, uint16_
 {
     if (elements <= 0 || elements % kBlock != 0)
         return hipErrorInvalidValue;
+    if (elements >= kWideElements && aligned_to(x, 16) && aligned_to(q, 8)) {
+        hipLaunchKernelGGL(quantize_rows_wide_kernel, dim3(blocks_for(elements, 8 * kThreads)),
+                           dim3(kThreads), 0, stream, x, elements, q, scales);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(quantize_rows_kernel, dim3(blocks_for(elements, kThreads)), dim3(kThreads),
                        0, stream, x, elements, q, scales);
     return hipGetLastError();
@@ -937,6 +1061,13 @@ hipError_t launch_embed(const uint32_t *tokens, const int *pos_ptr, int rows,
 {
     if (rows <= 0 || width <= 0 || width % kBlock != 0)
         return hipErrorInvalidValue;
+    const int64_t elements = (int64_t) rows * width;
+    if (elements >= kWideElements && aligned_to(table, 8) && aligned_to(out, 16)) {
+        hipLaunchKernelGGL(embed_wide_kernel, dim3(blocks_for(elements / 8, kThreads)),
+                           dim3(kThreads), 0, stream, tokens, pos_ptr, table, (int64_t) vocab, width,
+                           scale, out, elements / 8);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(embed_kernel, dim3(blocks_for(width, kThreads), rows), dim3(kThreads), 0,
                        stream, tokens, pos_ptr, nullptr, (int64_t) 0, table, (int64_t) vocab, width,
                        scale, out, nullptr, nullptr, 0, nullptr);
@@ -1172,6 +1303,12 @@ hipError_t launch_geglu(const float *fused, int rows, int intermediate, float *o
 {
     if (rows <= 0 || intermediate <= 0 || intermediate % kBlock != 0)
         return hipErrorInvalidValue;
+    if ((int64_t) rows * intermediate >= kWideElements && aligned_to(fused, 16)
+        && aligned_to(out, 16) && aligned_to(q8, 8)) {
+        hipLaunchKernelGGL(geglu_wide_kernel, dim3(blocks_for(intermediate, 8 * kThreads), rows),
+                           dim3(kThreads), 0, stream, fused, rows, intermediate, out, q8);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(geglu_kernel, dim3(blocks_for(intermediate, kThreads), rows),
                        dim3(kThreads), 0, stream, fused, rows, intermediate, out, q8);
     return hipGetLastError();

@@ -787,24 +787,27 @@ __global__ __launch_bounds__(kThreads) void mqa_partial_kernel(
     }
 }
 
-// Merge: a workgroup takes 512 channels of a query row, two a thread.  Lane s
+// Merge: a workgroup of T threads takes T C channels of a query row, C a
+// thread.  Lane s
 // of a wave holds split s's maximum and sum of a head, so the row's maximum,
 // the splits' factors and their total take a few lane exchanges, while the
 // first splits' channels are on their way; every split's channel is then
 // scaled and added in split order, divided by the total, rounded to fp32 and
 // optionally quantized.  (One workgroup a row, whose threads walked the 64
-// splits three times through memory, took 57 us for a row of 8000 keys.)
+// splits three times through memory, took 57 us for a row of 8000 keys.)  Few
+// rows take one-wave workgroups of 64 channels, so a row's partials come over
+// many compute units (63 splits of one row: 9.5 -> 5.2 us); many rows 512
+// channels a workgroup, which start fewer and share the factors.
 // tiled: the rows' splits are launch_tiled_attention's (rows it finished
 // itself are left alone), else mqa_partial_kernel's.
-constexpr int kMergeBatch = 8;
-constexpr int kMergeChannels = 2 * kThreads;
-
-__global__ __launch_bounds__(kThreads) void mqa_merge_kernel(
+template <int T, int C>
+__global__ __launch_bounds__(T) void mqa_merge_kernel(
     int heads, int head_dim, const int *pos_ptr, int pos_value, const double *__restrict__ ws_o,
     const double *__restrict__ ws_ml, float *__restrict__ out, uint8_t *__restrict__ q8, int rows,
     int tiled, AttentionSplit split)
 {
     static_assert(kMaxSplits == 64, "a lane a split");
+    constexpr int kMergeBatch = C == 1 ? 32 : 8; // splits requested at once
     __shared__ double sFactor[kMaxHeads][kMaxSplits];
     __shared__ double sTotal[kMaxHeads];
     const int row = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -821,26 +824,26 @@ __global__ __launch_bounds__(kThreads) void mqa_merge_kernel(
         splits = (keyCount + perSplit - 1) / perSplit;
     }
     const int qWidth = heads * head_dim;
-    const int first = blockIdx.x * kMergeChannels, end = min(first + kMergeChannels, qWidth);
+    const int first = blockIdx.x * T * C, end = min(first + T * C, qWidth);
     const int h0 = first / head_dim, h1 = (end - 1) / head_dim;
     const int64_t slot = (int64_t) row * kMaxSplits;
     const double *o = ws_o + slot * qWidth;
-    int idx[2];
-    double part[2][kMergeBatch];
+    int idx[C];
+    double part[C][kMergeBatch];
     auto load = [&](int s0) {
 #pragma unroll
         for (int s = 0; s < kMergeBatch; ++s)
 #pragma unroll
-            for (int c = 0; c < 2; ++c) // clamped into range; not used past the ends
+            for (int c = 0; c < C; ++c) // clamped into range; not used past the ends
                 part[c][s] = o[(int64_t) min(s0 + s, splits - 1) * qWidth + min(idx[c], qWidth - 1)];
     };
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
-        idx[c] = first + c * kThreads + (int) threadIdx.x;
+    for (int c = 0; c < C; ++c)
+        idx[c] = first + c * T + (int) threadIdx.x;
     load(0);
 
     const bool live = lane < splits;
-    for (int h = h0 + wave; h <= h1; h += kThreads / 64) {
+    for (int h = h0 + wave; h <= h1; h += T / 64) {
         const double *ml = ws_ml + ((slot + (live ? lane : 0)) * heads + h) * 2;
         const double m = live ? ml[0] : -INFINITY, sum = ml[1];
         const double largest = wave_max(m);
@@ -852,23 +855,25 @@ __global__ __launch_bounds__(kThreads) void mqa_merge_kernel(
             sTotal[h - h0] = total;
     }
     __syncthreads();
-    double weighted[2] = {0.0, 0.0};
-    int head[2];
+    double weighted[C];
+    int head[C];
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int c = 0; c < C; ++c) {
+        weighted[c] = 0.0;
         head[c] = min(idx[c], qWidth - 1) / head_dim - h0;
+    }
     for (int s0 = 0; s0 < splits; s0 += kMergeBatch) {
         if (s0 > 0)
             load(s0);
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+        for (int c = 0; c < C; ++c)
 #pragma unroll
             for (int s = 0; s < kMergeBatch; ++s)
                 if (s0 + s < splits)
                     weighted[c] += part[c][s] * sFactor[head[c]][s0 + s];
     }
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < C; ++c) {
         if (idx[c] >= qWidth) // whole 32-lane groups where there is a q8
             continue;
         const float v = (float) (weighted[c] / sTotal[head[c]]);
@@ -1291,9 +1296,14 @@ hipError_t launch_mqa(const float *queries, int q_stride, const uint16_t *key_ca
         if (status != hipSuccess)
             return status;
     }
-    if (merges)
-        hipLaunchKernelGGL(mqa_merge_kernel, dim3(blocks_for(heads * head_dim, kMergeChannels), rows),
-                           dim3(kThreads), 0, stream, heads, head_dim, pos_ptr, pos_value, wsO, wsMl, out, q8, rows,
+    if (merges && rows <= 16)
+        hipLaunchKernelGGL((mqa_merge_kernel<64, 1>), dim3(blocks_for(heads * head_dim, 64), rows),
+                           dim3(64), 0, stream, heads, head_dim, pos_ptr, pos_value, wsO, wsMl, out,
+                           q8, rows, tiled ? 1 : 0, split);
+    else if (merges)
+        hipLaunchKernelGGL((mqa_merge_kernel<kThreads, 2>),
+                           dim3(blocks_for(heads * head_dim, 2 * kThreads), rows), dim3(kThreads), 0,
+                           stream, heads, head_dim, pos_ptr, pos_value, wsO, wsMl, out, q8, rows,
                            tiled ? 1 : 0, split);
     return hipGetLastError();
 }

@@ -431,7 +431,8 @@ AttentionSplit attention_split(int rows, int heads, int kv_heads, int keys)
     const int stride = (blocks + kSamples - 1) / kSamples, samples = (blocks + stride - 1) / stride;
     double least = 0.0;
     int chosen = 0;
-    for (int splits = 1, last = 0; splits <= kAttentionSplits; splits += 1 + splits / 4) {
+    for (int step = 1, last = 0; step < 2 * kAttentionSplits; step += 1 + step / 4) {
+        const int splits = std::min(step, kAttentionSplits);
         const int per = ((longest + splits - 1) / splits + 3) / 4 * 4;
         if (per == last)
             continue;

@@ -1196,8 +1196,6 @@ hipError_t launch_matvec(const uint8_t *x8, int64_t xElements, int xRow, const u
 {
     const int segments = (inner / kBlock + 63) / 64;
     if (segments <= 1) {
-        if (outputs >= 131072)
-            return matvec_with<8, 1, 1>(x8, xElements, xRow, w8, inner, outputs, y, residual, stream);
         if (outputs >= 16384)
             return matvec_with<4, 1, 1>(x8, xElements, xRow, w8, inner, outputs, y, residual, stream);
         return matvec_with<1, 1, 1>(x8, xElements, xRow, w8, inner, outputs, y, residual, stream);
@@ -1227,7 +1225,9 @@ hipError_t launch_q8_product(const uint8_t *x8, int x_rows_total, int x_row0, in
         || x_row0 < 0 || x_row0 + rows > x_rows_total || product_lds(1, inner) > kProductLdsLimit)
         return hipErrorInvalidValue;
     const int64_t xElements = (int64_t) x_rows_total * inner;
-    if (rows == 1)
+    // one row: whole weight rows a wave, but for a vocabulary-wide product, which
+    // the 16 x 32 MFMA tile streams faster (2048 -> 256000: 94 against 87 us)
+    if (rows == 1 && (outputs < 131072 || inner > 2048))
         return launch_matvec(x8, xElements, x_row0, w8, inner, outputs, y, residual, stream);
     // a few rows of a narrow product: whole weight rows a wave stream better
     // than the MFMA tiles do (2 rows of 16384 -> 2048: 13.4 against 19.3 us,

@@ -509,7 +509,9 @@ hipError_t launch_q8_gemm(const uint8_t *x8, int64_t x_elements, int x_row0, int
 
 bool q8_gemm_geglu_supported(int rows, int inner, int intermediate)
 {
-    return rows > 1 && inner % kBlock == 0 && intermediate % kBlock == 0;
+    // (a tile's up rows lie intermediate rows past its gate rows: a 32-bit offset)
+    return rows > 1 && inner % kBlock == 0 && intermediate % kBlock == 0
+           && ((int64_t) intermediate + 64) * inner < (int64_t(1) << 32);
 }
 
 hipError_t launch_q8_gemm_geglu(const uint8_t *x8, int64_t x_elements, int x_row0, int rows,

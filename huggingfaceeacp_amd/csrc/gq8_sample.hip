@@ -22,7 +22,9 @@
 //   sample_bins_kernel     the chunks' masses; the bins' counts and masses
 //   sample_gather_kernel   the candidates of the bins that a cut can reach,
 //                          bin after bin
-//   sample_draw_kernel     one workgroup: the cuts and the draw
+//   sample_draw_kernel     one workgroup: the cuts and the draw; where the
+//                          gathered candidates are few enough to rank at once,
+//                          from their running masses alone (28 -> 5 us there)
 // A bin's mass is summed as integers of 2^-32 and 2^-64, so it does not depend
 // on the order the atomics land in (and is within 2^-65 a candidate of exact);
 // the sums along the ranking are doubles, so only their rounding differs from
@@ -31,7 +33,8 @@
 //
 // The launches are bound by their chains (a read of the chunk's 16 KB, the
 // atomics, the scans), not by the row's 1 MB.  A row of 256 000 normal logits
-// (sigma 3) at temperature 0.8, top-k 40, top-p 0.95: 69 us; the eight-pass
+// (sigma 3) at temperature 0.8, top-k 40, top-p 0.95: 46 us (4, 13, 12
+// and 5 in the kernels); the eight-pass
 // radix sort of the row, its one-workgroup scans and the draw over the ranked
 // row had taken 811.
 #include "gq8_device.hpp"
@@ -60,9 +63,17 @@ struct ChunkState {
     int unused;
 };
 
+// What the gather leaves for the draw.
+struct Gathered {
+    double total; // the row's mass
+    uint32_t count;
+    uint32_t unused;
+};
+
 struct SampleWorkspace {
     ChunkState *chunks;
     ChunkState *row;    // the whole row's
+    Gathered *summary;
     uint32_t *counts;   // of the bins
     uint32_t *cursors;  // candidates of a bin gathered so far
     uint64_t *massHi;   // multiples of 2^-32
@@ -266,6 +277,21 @@ struct Candidate {
     double massThrough;
 };
 
+// Ranks the candidates of rs.keys[0, n), n <= kRankCap, into rs.sorted (each
+// thread's takes its place among the others).
+__device__ inline void rank_candidates(RankShared &rs, uint32_t n)
+{
+    const uint32_t t = threadIdx.x;
+    if (t < n) {
+        const uint64_t mine = rs.keys[t];
+        uint32_t rank = 0;
+        for (uint32_t i = 0; i < n; ++i)
+            rank += rs.keys[i] < mine ? 1u : 0u;
+        rs.sorted[rank] = mine;
+    }
+    __syncthreads();
+}
+
 // The place's candidate among those of `span` (contiguous in `keys`).
 __device__ inline Candidate locate(const uint64_t *keys, Span span, const Place &place,
                                    double inverse, double top, BinShared &bs, RankShared &rs)
@@ -348,14 +374,7 @@ __device__ inline Candidate locate(const uint64_t *keys, Span span, const Place 
     }
     __syncthreads();
     const uint32_t n = span.count;
-    if (t < (int) n) {
-        const uint64_t mine = rs.keys[t];
-        uint32_t rank = 0;
-        for (uint32_t i = 0; i < n; ++i)
-            rank += rs.keys[i] < mine ? 1u : 0u;
-        rs.sorted[rank] = mine;
-    }
-    __syncthreads();
+    rank_candidates(rs, n);
     double weight = 0.0;
     if (t < (int) n)
         weight = candidate_weight(logit_of_key(rs.sorted[t]), inverse, top);
@@ -593,7 +612,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_gather_kernel(SampleArg
     const bool byMass = kept == n && !row.bad && mt > 0.0;
     const Place end{byMass ? kReaches : kRank, (uint32_t) kept - 1u,
                     (double) a.top_p * mt * (1.0 + 1e-9)};
-    const int lastBin = find_bin(sh, end, 0u, 0.0).bin;
+    const Span lastSpan = find_bin(sh, end, 0u, 0.0);
+    const int lastBin = lastSpan.bin;
+    if (blockIdx.x == 0 && t == 0)
+        *w.summary = Gathered{mt, lastSpan.before + lastSpan.count, 0u};
     int bin[kChunkRounds];
     uint32_t place[kChunkRounds];
 #pragma unroll
@@ -689,6 +711,51 @@ __device__ inline int token_order_draw(const SampleArgs &a, const SampleWorkspac
     return sFirst == INT_MAX ? sLast : sFirst;
 }
 
+// The cuts and the draw where every gathered candidate fits one ranking (a
+// top-k of some hundred, a peaked row): their running masses once, then each
+// place by a comparison a candidate.
+__device__ inline uint32_t few_candidates_draw(const SampleArgs &a, const SampleWorkspace &w, int n,
+                                               double uniform, double inverse, double top,
+                                               RankShared &rs)
+{
+    const uint32_t t = threadIdx.x, count = w.summary->count;
+    if (t < count)
+        rs.keys[t] = w.gathered[t];
+    __syncthreads();
+    rank_candidates(rs, count);
+    const double weight = t < count ? candidate_weight(logit_of_key(rs.sorted[t]), inverse, top) : 0.0;
+    uint32_t cb, ct;
+    double before, all;
+    workgroup_scan(0u, weight, cb, before, ct, all, rs.scan);
+    const double through = before + weight;
+    if (t < count)
+        rs.masses[t] = through;
+    // the first candidate that holds a place, `count` where none does
+    auto first = [&](const Place &place) {
+        __syncthreads(); // (also: the masses are in)
+        if (t == 0)
+            rs.found = count;
+        __syncthreads();
+        if (t < count && place.here(t + 1, through))
+            atomicMin(&rs.found, t);
+        __syncthreads();
+        return rs.found;
+    };
+    __syncthreads();
+    uint32_t kept = (uint32_t) first_kept(a, n);
+    double mass = kept < (uint32_t) n ? rs.masses[kept - 1] : w.summary->total;
+    if (a.top_p < 1.f) {
+        const uint32_t at = first(Place{kReaches, 0u, (double) a.top_p * mass});
+        if (at + 1 < kept) {
+            kept = min(at + 1, count); // the last gathered where rounding leaves none
+            mass = rs.masses[kept - 1];
+        }
+    }
+    kept = min(kept, count);
+    const uint32_t at = first(Place{kPasses, 0u, uniform * mass});
+    return (uint32_t) rs.sorted[at < kept ? at : kept - 1];
+}
+
 __global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(SampleArgs a, SampleWorkspace w)
 {
     __shared__ BinShared bins;
@@ -702,6 +769,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(SampleArgs 
     if (n > 0 && !cut(a, n)) {
         const int at = row.bad ? -1 : token_order_draw(a, w, uniform, inverse, top, bins.scan);
         chosen = (uint32_t) (at >= 0 ? at : row.last);
+    } else if (n > 0 && !row.bad && w.summary->total > 0.0 && w.summary->count <= (uint32_t) kRankCap) {
+        chosen = few_candidates_draw(a, w, n, uniform, inverse, top, ranks);
     } else if (n > 0) {
         load_bins(w, bins);
         uint32_t cb, ct;
@@ -769,6 +838,7 @@ SampleWorkspace carve(void *workspace, int vocab)
         return at;
     };
     w.row = reinterpret_cast<ChunkState *>(take(sizeof(ChunkState)));
+    w.summary = reinterpret_cast<Gathered *>(take(sizeof(Gathered)));
     w.chunks = reinterpret_cast<ChunkState *>(take(w.chunkCount * sizeof(ChunkState)));
     w.counts = reinterpret_cast<uint32_t *>(take(kBins * sizeof(uint32_t)));
     w.cursors = reinterpret_cast<uint32_t *>(take(kBins * sizeof(uint32_t)));
@@ -784,7 +854,7 @@ size_t sample_workspace_bytes(int vocab)
 {
     if (vocab <= 0)
         return 0;
-    return align256(sizeof(ChunkState)) + align256(sample_chunks(vocab) * sizeof(ChunkState))
+    return align256(sizeof(ChunkState)) + align256(sizeof(Gathered)) + align256(sample_chunks(vocab) * sizeof(ChunkState))
            + 2 * align256(kBins * sizeof(uint32_t)) + 2 * align256(kBins * sizeof(uint64_t))
            + align256((size_t) vocab * sizeof(uint64_t)) + 256; // and its alignment
 }

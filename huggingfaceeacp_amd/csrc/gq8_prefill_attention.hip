@@ -408,7 +408,7 @@ bool tiled_attention_supported(int head_dim, const float *queries, int q_stride,
 // of a sweep at eight heads of 256 over one KV head (rows 1 .. 2048, 0 .. 8000
 // keys before them).  Microseconds there, one workgroup a block -> split: 333
 // rows behind 700 keys 99 -> 77, 128 behind 4000 352 -> 105, 16 behind 8000
-// 672 -> 42, one row of 8000 keys 680 -> 31 (110 in mqa_partial_kernel and its
+// 672 -> 42, one row of 8000 keys 680 -> 27 (110 in mqa_partial_kernel and its
 // former merge); 512 rows behind 512 keys and 2048 alone stay whole (94, 330).
 AttentionSplit attention_split(int rows, int heads, int kv_heads, int keys)
 {

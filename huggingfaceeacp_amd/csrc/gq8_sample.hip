@@ -34,9 +34,8 @@
 // The launches are bound by their chains (a read of the chunk's 16 KB, the
 // atomics, the scans), not by the row's 1 MB.  A row of 256 000 normal logits
 // (sigma 3) at temperature 0.8, top-k 40, top-p 0.95: 46 us (4, 13, 12
-// and 5 in the kernels); the eight-pass
-// radix sort of the row, its one-workgroup scans and the draw over the ranked
-// row had taken 811.
+// and 5 in the kernels); the eight-pass radix sort of the row, its
+// one-workgroup scans and the draw over the ranked row had taken 811.
 #include "gq8_device.hpp"
 #include "gq8_kernels.hpp"
 #include "gq8_numerics.hpp"

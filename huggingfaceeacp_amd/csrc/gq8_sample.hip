@@ -291,7 +291,10 @@ __device__ inline void rank_candidates(RankShared &rs, uint32_t n)
     __syncthreads();
 }
 
-// The place's candidate among those of `span` (contiguous in `keys`).
+// The place's candidate among those of `span` (contiguous in `keys`).  Keys
+// are distinct, so every pass of the search leaves fewer of them; it ends on
+// any content (the key range at least halves a pass) and ranks no more than
+// rs.keys holds.
 __device__ inline Candidate locate(const uint64_t *keys, Span span, const Place &place,
                                    double inverse, double top, BinShared &bs, RankShared &rs)
 {
@@ -320,6 +323,8 @@ __device__ inline Candidate locate(const uint64_t *keys, Span span, const Place 
         __syncthreads();
         low = rs.low;
         high = rs.high;
+        if (low >= high)
+            break;
         int shift = 0;
         while (((high - low) >> shift) >= (uint64_t) kBins)
             ++shift;
@@ -368,11 +373,14 @@ __device__ inline Candidate locate(const uint64_t *keys, Span span, const Place 
     __syncthreads();
     for (uint32_t i = t; i < size; i += kSampleThreads) {
         const uint64_t k = keys[i];
-        if (k >= low && k <= high)
-            rs.keys[atomicAdd(&rs.gathered, 1u)] = k;
+        if (k >= low && k <= high) {
+            const uint32_t at = atomicAdd(&rs.gathered, 1u);
+            if (at < (uint32_t) kRankCap)
+                rs.keys[at] = k;
+        }
     }
     __syncthreads();
-    const uint32_t n = span.count;
+    const uint32_t n = min(rs.gathered, (uint32_t) kRankCap);
     rank_candidates(rs, n);
     double weight = 0.0;
     if (t < (int) n)
@@ -778,13 +786,13 @@ __global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(SampleArgs 
         // the bin of a place, and the candidate in it (its bin's gathered
         // candidates; `locate` may use the bins' space, which is then loaded
         // again)
-        auto find = [&](const Place &place) {
-            const Span span = find_bin(bins, place, 0u, 0.0);
+        auto find_in = [&](const Span &span, const Place &place) {
             const Candidate c = locate(w.gathered + span.before, span, place, inverse, top, bins, ranks);
             if (span.count > (uint32_t) kRankCap)
                 load_bins(w, bins);
             return c;
         };
+        auto find = [&](const Place &place) { return find_in(find_bin(bins, place, 0u, 0.0), place); };
         const bool sums = !row.bad && all > 0.0; // else no running mass is a number
         int kept = first_kept(a, n);
         double mass = all;
@@ -806,9 +814,16 @@ __global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(SampleArgs 
         }
         bool drawn = false;
         if (sums) {
-            const Candidate c = find(Place{kPasses, 0u, uniform * mass});
-            drawn = (int) c.rank < kept;
-            chosen = c.token;
+            // the bins' running masses and `mass` are different sums of the same
+            // weights: the largest draws may lie past the last kept candidate's
+            // bin, where nothing is kept (or gathered)
+            const Place place{kPasses, 0u, uniform * mass};
+            const Span span = find_bin(bins, place, 0u, 0.0);
+            if ((int) span.before < kept) {
+                const Candidate c = find_in(span, place);
+                drawn = (int) c.rank < kept;
+                chosen = c.token;
+            }
         }
         if (!drawn) {
             if (!known)

@@ -1,13 +1,14 @@
 """The sampler's bins at their edges, against the oracle's draws: rows whose
 candidates crowd one bin (equal logits, a narrow spread), rows spread past the
 bins' range (low temperatures, infinitely unlikely tokens), vocabularies around
-a chunk's and a bin search's sizes, and cuts that keep one, all or almost all
-candidates."""
+a chunk's and a bin search's sizes, cuts that keep one, all or almost all
+candidates, and the largest draw there is."""
 import numpy as np
 import pytest
 
+import oracle as O
 from huggingfaceeacp_amd import gemma_q8 as G
-from test_gpu_sampling import agree
+from test_gpu_sampling import DeviceSampler, agree
 
 pytestmark = pytest.mark.gpu
 S = G.SamplingOptions
@@ -70,3 +71,31 @@ def test_a_row_without_a_number_keeps_its_last_candidate(torch_cuda):
         assert sample(S(1.0, top_k=k_th)) == vocab - (k_th - 1)
         assert sample(S(1.0, top_p=0.5)) == 0
         assert sample(S(1.0)) == vocab - 1
+
+
+def drawn(torch, row, options, uniform):
+    """(the device's id, the oracle's) of one given draw."""
+    row = np.ascontiguousarray(row, dtype=np.float32)
+    want = O.lib().gor_sample(O.ptr(row), None, row.size, options.temperature, options.top_k,
+                              options.top_p, uniform)
+    sampler = DeviceSampler(torch, row.size)
+    sampler.workspace.zero_()
+    return sampler.sample(torch.from_numpy(row).cuda(), None, options, uniform), int(want)
+
+
+@pytest.mark.parametrize("seed", [7, 11, 12, 14, 16])
+def test_largest_draw_keeps_to_the_kept_candidates(torch_cuda, seed):
+    """The draw 1 - 2^-53 over 1000 kept candidates that share a bin of the
+    score, or fill some of them, with thousands more far below.  At these seeds
+    the crowded bin's running mass rounds below the draw's target (the sums
+    restated in numpy), so the place lies past every kept candidate: the
+    last of them is the answer (Sampler.cpp:196-213)."""
+    for spread in (0.012, 0.2):
+        near = (-np.random.default_rng(seed).random(1000) * spread).astype(np.float32)
+        near[0] = 0
+        row = np.concatenate([near, np.full(5000, -20.0, np.float32)])
+        for options in (S(1.0, top_k=1000), S(1.0, top_k=700), S(1.0, top_p=0.9),
+                        S(1.0, top_k=1000, top_p=0.97)):
+            for uniform in (1.0 - 2.0 ** -53, 1.0 - 2.0 ** -52, 0.0):
+                got, want = drawn(torch_cuda, row, options, uniform)
+                assert got == want, (spread, options, uniform)

@@ -362,8 +362,8 @@ __device__ inline Candidate locate(const uint64_t *keys, Span span, const Place 
         __syncthreads();
         span = find_bin(bs, place, span.before, span.massBefore);
         low += (uint64_t) span.bin << shift;
-        const uint64_t end = low + ((1ull << shift) - 1);
-        high = end < high ? end : high;
+        const uint64_t reach = (1ull << shift) - 1; // low + reach may pass 2^64
+        high = high - low < reach ? high : low + reach;
     }
     // few enough: each thread's candidate takes its place among the others
     if (t == 0) {

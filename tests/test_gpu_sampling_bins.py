@@ -99,3 +99,17 @@ def test_largest_draw_keeps_to_the_kept_candidates(torch_cuda, seed):
             for uniform in (1.0 - 2.0 ** -53, 1.0 - 2.0 ** -52, 0.0):
                 got, want = drawn(torch_cuda, row, options, uniform)
                 assert got == want, (spread, options, uniform)
+
+
+def test_last_ranking_key_ends_the_search_range(torch_cuda):
+    """More than a ranking's worth of -inf logits and, behind them all, a NaN
+    with every bit set, whose ranking key has the largest upper word: the
+    range of the last bin searched ends there and does not wrap.  No
+    running mass is a number, so the last of the ranking is kept."""
+    row = np.linspace(-3, 3, 3000).astype(np.float32)
+    row[10:800] = -np.inf
+    row.view(np.uint32)[5] = 0xFFFFFFFF
+    sampler = DeviceSampler(torch_cuda, row.size)
+    dev = torch_cuda.from_numpy(row).cuda()
+    for options in (S(1.0, top_p=0.9), S(0.5, top_k=3000, top_p=0.5)):
+        assert sampler.sample(dev, None, options, 0.25) == 5

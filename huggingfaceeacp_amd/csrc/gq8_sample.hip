@@ -58,8 +58,9 @@ struct ChunkState {
     double mass;    // of its weights, in a fixed order
     int count;      // unmasked tokens
     int last;       // the last of them, -1 where there is none
-    int bad;        // a NaN or +infinite logit among them: no sum of weights is a number
-    int unused;
+    int bad;        // one that ranks before every number (a +infinity, a NaN of clear sign): no
+                    // sum along the ranking is a number
+    int nans;       // NaNs with the sign set, which rank after every number
 };
 
 // What the gather leaves for the draw.
@@ -119,6 +120,12 @@ __device__ inline double candidate_weight(float logit, double inverse, double to
     return exp(candidate_score(logit, inverse) - top);
 }
 
+// A NaN with the sign set: ranked after every number.
+__device__ inline bool nan_behind(float logit)
+{
+    return logit != logit && (__float_as_uint(logit) >> 31);
+}
+
 // The bin of a score `distance` = top - score below the largest: 64 a unit up
 // to 16, then 64 an octave (the top bits of the distance as a float), the last
 // one for all that lie past 2^20.  Never decreasing in the distance.  A
@@ -128,7 +135,7 @@ __device__ inline int distance_bin(float logit, double inverse, double top)
 {
     const double distance = top - candidate_score(logit, inverse);
     if (!(distance >= 0.0))
-        return logit != logit && (__float_as_uint(logit) >> 31) ? kBins - 1 : 0;
+        return nan_behind(logit) ? kBins - 1 : 0;
     if (distance < 16.0)
         return (int) (distance * 64.0);
     const float f = (float) fmin(distance, 1e30);
@@ -136,9 +143,10 @@ __device__ inline int distance_bin(float logit, double inverse, double top)
     return min(kBins / 2 + octaves, kBins - 1);
 }
 
+// A NaN counts as nothing: it ranks after every number whose sum is used.
 __device__ inline void split_mass(double w, uint64_t &hi, uint64_t &lo)
 {
-    const double scaled = w * 4294967296.0;
+    const double scaled = fmax(w, 0.0) * 4294967296.0;
     const double whole = floor(scaled);
     hi = (uint64_t) whole;
     lo = (uint64_t) rint((scaled - whole) * 4294967296.0);
@@ -408,12 +416,13 @@ __device__ inline Candidate locate(const uint64_t *keys, Span span, const Place 
 __device__ inline ChunkState row_state(const ChunkState *chunks, int count)
 {
     __shared__ double sLargest[kSampleWaves];
-    __shared__ int sCount, sLast, sBad;
+    __shared__ int sCount, sLast, sBad, sNans;
     const int t = threadIdx.x;
     if (t == 0) {
         sCount = 0;
         sLast = -1;
         sBad = 0;
+        sNans = 0;
     }
     __syncthreads();
     double largest = -DBL_MAX;
@@ -424,6 +433,8 @@ __device__ inline ChunkState row_state(const ChunkState *chunks, int count)
         atomicMax(&sLast, c.last);
         if (c.bad)
             atomicOr(&sBad, 1);
+        if (c.nans)
+            atomicAdd(&sNans, c.nans);
     }
     largest = wave_max_d(largest);
     if ((t & 63) == 0)
@@ -436,6 +447,7 @@ __device__ inline ChunkState row_state(const ChunkState *chunks, int count)
     s.count = sCount;
     s.last = sLast;
     s.bad = sBad;
+    s.nans = sNans;
     return s;
 }
 
@@ -447,7 +459,7 @@ __device__ inline bool masked(const SampleArgs &a, int token)
 __global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a, SampleWorkspace w)
 {
     __shared__ double sLargest[kSampleWaves];
-    __shared__ int sCount, sLast, sBad;
+    __shared__ int sCount, sLast, sBad, sNans;
     const int t = threadIdx.x;
     for (int b = blockIdx.x * kSampleThreads + t; b < kBins; b += gridDim.x * kSampleThreads) {
         w.counts[b] = 0u;
@@ -459,6 +471,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a
         sCount = 0;
         sLast = -1;
         sBad = 0;
+        sNans = 0;
     }
     __syncthreads();
     const double inverse = 1.0 / (double) a.temperature;
@@ -472,14 +485,16 @@ __global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a
         logit[r] = a.logits[e < a.vocab ? e : 0];
     }
     double largest = -DBL_MAX;
-    int count = 0, last = -1, bad = 0;
+    int count = 0, last = -1, bad = 0, nans = 0;
 #pragma unroll
     for (int r = 0; r < kChunkRounds; ++r)
         if (live[r]) {
             largest = fmax(largest, candidate_score(logit[r], inverse));
             ++count;
             last = (int) (first + r * kSampleThreads);
-            bad |= !(logit[r] < INFINITY);
+            const bool behind = nan_behind(logit[r]);
+            nans += behind;
+            bad |= !(logit[r] < INFINITY) && !behind;
         }
     largest = wave_max_d(largest);
     const double deepest = wave_max_d((double) last); // exact: below 2^31
@@ -487,6 +502,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a
     for (int d = 32; d >= 1; d >>= 1)
         count += __shfl_xor(count, d);
     const bool anyBad = __any(bad) != 0;
+    if (nans)
+        atomicAdd(&sNans, nans);
     if ((t & 63) == 0) { // one atomic a wave
         sLargest[t >> 6] = largest;
         atomicAdd(&sCount, count);
@@ -499,7 +516,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a
         double m = -DBL_MAX;
         for (int i = 0; i < kSampleWaves; ++i)
             m = fmax(m, sLargest[i]);
-        w.chunks[blockIdx.x] = ChunkState{m, 0.0, sCount, sLast, sBad, 0};
+        w.chunks[blockIdx.x] = ChunkState{m, 0.0, sCount, sLast, sBad, sNans};
     }
 }
 
@@ -584,6 +601,12 @@ __device__ inline int first_kept(const SampleArgs &a, int n)
     return a.top_k > 0 && a.top_k < n ? a.top_k : n;
 }
 
+// Whether the weights of the first `kept` ranked candidates are numbers.
+__device__ inline bool weights_are_numbers(const ChunkState &row, int kept)
+{
+    return !row.bad && kept <= row.count - row.nans;
+}
+
 __global__ __launch_bounds__(kSampleThreads) void sample_gather_kernel(SampleArgs a, SampleWorkspace w)
 {
     __shared__ BinShared sh;
@@ -616,7 +639,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_gather_kernel(SampleArg
     sMine[2 * t] = 0u;
     sMine[2 * t + 1] = 0u;
     const int kept = first_kept(a, n);
-    const bool byMass = kept == n && !row.bad && mt > 0.0;
+    const bool byMass = kept == n && weights_are_numbers(row, n) && mt > 0.0;
     const Place end{byMass ? kReaches : kRank, (uint32_t) kept - 1u,
                     (double) a.top_p * mt * (1.0 + 1e-9)};
     const Span lastSpan = find_bin(sh, end, 0u, 0.0);
@@ -774,9 +797,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(SampleArgs 
     const int n = row.count;
     uint32_t chosen = 0;
     if (n > 0 && !cut(a, n)) {
-        const int at = row.bad ? -1 : token_order_draw(a, w, uniform, inverse, top, bins.scan);
+        const int at = !weights_are_numbers(row, n) ? -1 : token_order_draw(a, w, uniform, inverse, top, bins.scan);
         chosen = (uint32_t) (at >= 0 ? at : row.last);
-    } else if (n > 0 && !row.bad && w.summary->total > 0.0 && w.summary->count <= (uint32_t) kRankCap) {
+    } else if (n > 0 && weights_are_numbers(row, first_kept(a, n)) && w.summary->total > 0.0
+               && w.summary->count <= (uint32_t) kRankCap) {
         chosen = few_candidates_draw(a, w, n, uniform, inverse, top, ranks);
     } else if (n > 0) {
         load_bins(w, bins);
@@ -793,8 +817,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(SampleArgs 
             return c;
         };
         auto find = [&](const Place &place) { return find_in(find_bin(bins, place, 0u, 0.0), place); };
-        const bool sums = !row.bad && all > 0.0; // else no running mass is a number
         int kept = first_kept(a, n);
+        const bool sums = weights_are_numbers(row, kept) && all > 0.0; // else no running mass is a number
         double mass = all;
         Candidate end{};
         bool known = false; // `end` is the last kept candidate

@@ -113,3 +113,30 @@ def test_last_ranking_key_ends_the_search_range(torch_cuda):
     dev = torch_cuda.from_numpy(row).cuda()
     for options in (S(1.0, top_p=0.9), S(0.5, top_k=3000, top_p=0.5)):
         assert sampler.sample(dev, None, options, 0.25) == 5
+
+
+@pytest.mark.parametrize("count", [1, 700])
+def test_nans_behind_the_kept_candidates_weigh_nothing(torch_cuda, count):
+    """NaNs with the sign set rank after every number, so a top-k that keeps
+    numbers alone draws as if they were -inf; one that keeps the first of
+    them has no sums that are numbers and takes its last candidate."""
+    vocab = 3000
+    rng = np.random.default_rng(count)
+    row = rng.normal(0, 2, vocab).astype(np.float32)
+    at = np.sort(rng.choice(vocab, count, replace=False))
+    numbers, bits = row.copy(), row.copy()
+    numbers[at] = -np.inf
+    bits.view(np.uint32)[at] = 0xFFC00000
+    dev = torch_cuda.from_numpy(bits).cuda()
+    sampler = DeviceSampler(torch_cuda, vocab)
+    for options in (S(1.0, top_k=40, seed=51), S(0.8, top_k=40, top_p=0.9, seed=52),
+                    S(1.0, top_k=vocab - count, seed=53),
+                    S(1.0, top_k=vocab - count, top_p=0.95, seed=54)):
+        ref = O.Sampler(options.temperature, options.top_k, options.top_p, options.seed)
+        for uniform in O.uniform_draws(options.seed, 20):
+            assert sampler.sample(dev, None, options, uniform) == ref.sample(numbers), (options, uniform)
+    if count > 1:
+        for options in (S(1.0, top_k=vocab - count + 1), S(1.0, top_k=vocab - count + 1, top_p=0.5)):
+            assert sampler.sample(dev, None, options, 0.25) == at[0]
+    assert sampler.sample(dev, None, S(1.0, top_p=0.5), 0.25) == at[-1]
+    assert sampler.sample(dev, None, S(1.0), 0.25) == vocab - 1

@@ -99,7 +99,15 @@ __device__ inline double candidate_score(float logit, double inverse)
     return s == 0.0 ? 0.0 : s;
 }
 
-// The ranking key of a candidate: descending in the logit (the score is
+// A token's logit.  At an infinite temperature the scores are logit * 0, so
+// the logits are taken as that: they tie (an infinity is then a NaN).
+__device__ inline float row_logit(const SampleArgs &a, int64_t token)
+{
+    const float logit = a.logits[token];
+    return a.temperature < INFINITY ? logit : logit * 0.f;
+}
+
+// The ranking key of a candidate: descending in row_logit (the score is
 // strictly increasing in it), then ascending in the token.
 __device__ inline uint64_t ranking_key(float logit, uint32_t token)
 {
@@ -482,7 +490,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a
     for (int r = 0; r < kChunkRounds; ++r) {
         const int64_t e = first + r * kSampleThreads;
         live[r] = e < a.vocab && !masked(a, (int) e);
-        logit[r] = a.logits[e < a.vocab ? e : 0];
+        logit[r] = row_logit(a, e < a.vocab ? e : 0);
     }
     double largest = -DBL_MAX;
     int count = 0, last = -1, bad = 0, nans = 0;
@@ -534,7 +542,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_bins_kernel(SampleArgs 
     for (int r = 0; r < kChunkRounds; ++r) {
         const int64_t e = first + r * kSampleThreads;
         live[r] = e < a.vocab && !masked(a, (int) e);
-        logit[r] = a.logits[e < a.vocab ? e : 0];
+        logit[r] = row_logit(a, e < a.vocab ? e : 0);
     }
     if (ranked)
         for (int b = t; b < kBins; b += kSampleThreads) {
@@ -619,7 +627,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_gather_kernel(SampleArg
     for (int r = 0; r < kChunkRounds; ++r) {
         const int64_t e = first + r * kSampleThreads;
         live[r] = e < a.vocab && !masked(a, (int) e);
-        logit[r] = a.logits[e < a.vocab ? e : 0];
+        logit[r] = row_logit(a, e < a.vocab ? e : 0);
     }
     const ChunkState row = *w.row;
     const int n = row.count;
@@ -716,7 +724,7 @@ __device__ inline int token_order_draw(const SampleArgs &a, const SampleWorkspac
     for (int r = 0; r < kChunkRounds; ++r) {
         const int64_t e = first + r;
         const bool live = e < a.vocab && !masked(a, (int) e);
-        weight[r] = live ? candidate_weight(a.logits[e], inverse, top) : 0.0;
+        weight[r] = live ? candidate_weight(row_logit(a, e), inverse, top) : 0.0;
         sum += weight[r];
         last = weight[r] > 0.0 ? (int) e : last;
     }

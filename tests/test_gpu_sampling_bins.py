@@ -140,3 +140,14 @@ def test_nans_behind_the_kept_candidates_weigh_nothing(torch_cuda, count):
             assert sampler.sample(dev, None, options, 0.25) == at[0]
     assert sampler.sample(dev, None, S(1.0, top_p=0.5), 0.25) == at[-1]
     assert sampler.sample(dev, None, S(1.0), 0.25) == vocab - 1
+
+
+@pytest.mark.parametrize("vocab", [40, 3000, 60000])
+def test_infinite_temperature_ranks_by_token(torch_cuda, vocab):
+    """1 / temperature is zero: every score ties, whatever the logits."""
+    row = np.random.default_rng(vocab).normal(0, 2, vocab).astype(np.float32)
+    inf = float("inf")
+    for options in (S(inf, top_k=5, seed=61), S(inf, top_k=vocab - 1, top_p=0.47, seed=62),
+                    S(inf, top_p=0.9, seed=63), S(inf, seed=64)):
+        got = agree(torch_cuda, row, options, draws=12)
+        assert options.top_k != 5 or max(got) < 5

@@ -11,12 +11,14 @@
 //
 // Nothing sorts the row.  Each step needs one place in the ranking (the k-th
 // candidate, the one that reaches a mass), so the row is spread over 2048
-// bins of the distance to the largest score, whose order is the ranking's; a
+// bins (BinRule) whose order is the ranking's; a
 // scan of the bins' counts and masses gives the bin that holds the place, and
-// that bin's candidates alone are ranked.  A bin past kRankCap candidates is
-// spread over 2048 bins again, of the range its (score, token) keys cover,
-// until few enough are left, so a flat row or one of equal logits costs a few
-// passes over its own candidates.  Four launches:
+// that bin's candidates alone are ranked.  The bins' width follows the row's
+// spread, so a flat row or one of equal logits fills them too.  A bin past
+// kRankCap candidates (a crowd of near ties below an outlier) is spread over
+// 2048 bins again, of the range its (score, token) keys cover, until few
+// enough are left: some passes of one workgroup over its candidates.  Four
+// launches:
 //   sample_max_kernel      each chunk's largest score, unmasked count and last
 //                          unmasked token; the bins cleared
 //   sample_bins_kernel     the chunks' masses; the bins' counts and masses
@@ -35,7 +37,10 @@
 // atomics, the scans), not by the row's 1 MB.  A row of 256 000 normal logits
 // (sigma 3) at temperature 0.8, top-k 40, top-p 0.95: 46 us (4, 13, 12
 // and 5 in the kernels); the eight-pass radix sort of the row, its
-// one-workgroup scans and the draw over the ranked row had taken 811.
+// one-workgroup scans and the draw over the ranked row had taken 811.  256 000
+// equal logits with these options: 56 us (the sort 724; with bins of one width
+// for all rows, all candidates in one of them, 2300).  255 999 logits within
+// 1e-5 of each other below an outlier, top-k 1000: 715 (the sort 728).
 #include "gq8_device.hpp"
 #include "gq8_kernels.hpp"
 #include "gq8_numerics.hpp"
@@ -54,7 +59,7 @@ constexpr int kBins = 2 * kSampleThreads;                      // two a thread i
 constexpr int kRankCap = 512;                                  // candidates ranked by counting
 
 struct ChunkState {
-    double largest; // of the chunk's unmasked scores, -DBL_MAX where there is none
+    float largest, smallest; // of the chunk's unmasked row_logits but NaNs (-inf, inf where there is none)
     double mass;    // of its weights, in a fixed order
     int count;      // unmasked tokens
     int last;       // the last of them, -1 where there is none
@@ -123,6 +128,13 @@ __device__ inline float logit_of_key(uint64_t key)
     return __uint_as_float(u);
 }
 
+// The row's largest score, which weighs 1 (the lowest double where all are
+// -infinite).
+__device__ inline double top_score(const ChunkState &row, double inverse)
+{
+    return fmax(-DBL_MAX, candidate_score(row.largest, inverse));
+}
+
 __device__ inline double candidate_weight(float logit, double inverse, double top)
 {
     return exp(candidate_score(logit, inverse) - top);
@@ -134,16 +146,38 @@ __device__ inline bool nan_behind(float logit)
     return logit != logit && (__float_as_uint(logit) >> 31);
 }
 
-// The bin of a score `distance` = top - score below the largest: 64 a unit up
-// to 16, then 64 an octave (the top bits of the distance as a float), the last
-// one for all that lie past 2^20.  Never decreasing in the distance.  A
-// NaN: before every number with the sign clear, after with it set, as the
-// ranking key has it (an infinity's distance to itself is a NaN of clear sign).
-__device__ inline int distance_bin(float logit, double inverse, double top)
+// The bins of a row.  A score lies `distance` = top - score below the largest:
+// 64 bins a unit up to 16, then 64 an octave (the top bits of the distance as
+// a float), the last one for all that lie past 2^20.  Where all scores lie
+// within 8 of the largest, distances are scaled by a power of two to fill the
+// even bins, and where they tie, the bins go by token (`tokens` each): a flat
+// row's candidates do not crowd a few bins.
+struct BinRule {
+    double top, scale;
+    int tokens; // 0: by distance
+};
+
+__device__ inline BinRule bin_rule(const ChunkState &row, double inverse, int vocab)
 {
-    const double distance = top - candidate_score(logit, inverse);
+    BinRule rule{top_score(row, inverse), 1.0, 0};
+    const double range = rule.top - candidate_score(row.smallest, inverse);
+    if (range == 0.0)
+        rule.tokens = (vocab + kBins - 1) / kBins;
+    else if (range > 0.0 && range < 8.0)
+        rule.scale = ldexp(1.0, min(3 - ilogb(range), 1000));
+    return rule;
+}
+
+// Never decreasing along the ranking.  A NaN: before every number with the
+// sign clear, after with it set, as the ranking key has it (an infinity's
+// distance to itself is a NaN of clear sign).
+__device__ inline int candidate_bin(float logit, int token, double inverse, const BinRule &rule)
+{
+    const double distance = (rule.top - candidate_score(logit, inverse)) * rule.scale;
     if (!(distance >= 0.0))
         return nan_behind(logit) ? kBins - 1 : 0;
+    if (rule.tokens)
+        return token / rule.tokens;
     if (distance < 16.0)
         return (int) (distance * 64.0);
     const float f = (float) fmin(distance, 1e30);
@@ -277,6 +311,7 @@ __device__ inline Span find_bin(BinShared &sh, const Place &place, uint32_t befo
 }
 
 struct RankShared {
+    uint64_t massLo[kBins]; // `locate`: multiples of 2^-64 in a bin
     uint64_t keys[kRankCap], sorted[kRankCap];
     double masses[kRankCap];
     ScanShared scan;
@@ -307,6 +342,31 @@ __device__ inline void rank_candidates(RankShared &rs, uint32_t n)
     __syncthreads();
 }
 
+// use(key) for each of keys[0, size), eight loads a thread in flight.
+// kStretches: a thread takes a stretch of its own in place of every 1024th key.
+// The loads then touch a line a lane, but the gather leaves a bin's keys
+// about in token order, and where scores tie, neighbours share a bin of the
+// search, whose LDS atomics a whole wave would make one after another.
+template <bool kStretches, typename Use>
+__device__ inline void each_key(const uint64_t *keys, uint32_t size, Use use)
+{
+    constexpr uint32_t kLoads = 8;
+    constexpr uint32_t kStep = kStretches ? 1u : (uint32_t) kSampleThreads;
+    const uint32_t batches = (size + kLoads * kSampleThreads - 1) / (kLoads * kSampleThreads);
+    const uint32_t first = threadIdx.x * (kStretches ? kLoads * batches : 1u);
+    for (uint32_t n = 0; n < batches; ++n) {
+        const uint32_t i0 = first + n * kLoads * kStep;
+        uint64_t k[kLoads];
+#pragma unroll
+        for (uint32_t r = 0; r < kLoads; ++r)
+            k[r] = keys[min(i0 + r * kStep, size - 1)];
+#pragma unroll
+        for (uint32_t r = 0; r < kLoads; ++r)
+            if (i0 + r * kStep < size)
+                use(k[r]);
+    }
+}
+
 // The place's candidate among those of `span` (contiguous in `keys`).  Keys
 // are distinct, so every pass of the search leaves fewer of them; it ends on
 // any content (the key range at least halves a pass) and ranks no more than
@@ -323,17 +383,19 @@ __device__ inline Candidate locate(const uint64_t *keys, Span span, const Place 
             rs.low = ~0ull;
             rs.high = 0ull;
         }
-        for (int b = t; b < kBins; b += kSampleThreads)
+        for (int b = t; b < kBins; b += kSampleThreads) {
             bs.counts[b] = 0u;
+            bs.masses[b] = 0.0; // all bits clear
+            rs.massLo[b] = 0ull;
+        }
         __syncthreads();
         uint64_t lo = ~0ull, hi = 0ull;
-        for (uint32_t i = t; i < size; i += kSampleThreads) {
-            const uint64_t k = keys[i];
+        each_key<false>(keys, size, [&](uint64_t k) {
             if (k >= low && k <= high) {
                 lo = k < lo ? k : lo;
                 hi = k > hi ? k : hi;
             }
-        }
+        });
         atomicMin((unsigned long long *) &rs.low, (unsigned long long) lo);
         atomicMax((unsigned long long *) &rs.high, (unsigned long long) hi);
         __syncthreads();
@@ -344,37 +406,23 @@ __device__ inline Candidate locate(const uint64_t *keys, Span span, const Place 
         int shift = 0;
         while (((high - low) >> shift) >= (uint64_t) kBins)
             ++shift;
-        // a candidate's mass as integers, so the sums' order does not matter:
-        // the high part in masses, the low part below 2^-32 a second time round
-        uint64_t *parts = reinterpret_cast<uint64_t *>(bs.masses);
-        double total[2];
-        for (int part = 0; part < 2; ++part) {
-            for (int b = t; b < kBins; b += kSampleThreads)
-                parts[b] = 0ull;
-            __syncthreads();
-            for (uint32_t i = t; i < size; i += kSampleThreads) {
-                const uint64_t k = keys[i];
-                if (k < low || k > high)
-                    continue;
-                const int b = (int) ((k - low) >> shift);
-                uint64_t mh, ml;
-                split_mass(candidate_weight(logit_of_key(k), inverse, top), mh, ml);
-                atomicAdd((unsigned long long *) &parts[b], (unsigned long long) (part ? ml : mh));
-                if (part == 0)
-                    atomicAdd(&bs.counts[b], 1u);
-            }
-            __syncthreads();
-            if (part == 0) {
-                total[0] = (double) parts[2 * t] * 0x1p-32;
-                total[1] = (double) parts[2 * t + 1] * 0x1p-32;
-            } else {
-                total[0] += (double) parts[2 * t] * 0x1p-64;
-                total[1] += (double) parts[2 * t + 1] * 0x1p-64;
-            }
-            __syncthreads();
-        }
-        bs.masses[2 * t] = total[0];
-        bs.masses[2 * t + 1] = total[1];
+        // a candidate's mass as integers, so the sums' order does not matter
+        uint64_t *massHi = reinterpret_cast<uint64_t *>(bs.masses);
+        each_key<true>(keys, size, [&](uint64_t k) {
+            if (k < low || k > high)
+                return;
+            const int b = (int) ((k - low) >> shift);
+            uint64_t mh, ml;
+            split_mass(candidate_weight(logit_of_key(k), inverse, top), mh, ml);
+            atomicAdd(&bs.counts[b], 1u);
+            if (mh)
+                atomicAdd((unsigned long long *) &massHi[b], (unsigned long long) mh);
+            if (ml)
+                atomicAdd((unsigned long long *) &rs.massLo[b], (unsigned long long) ml);
+        });
+        __syncthreads();
+        for (int b = t; b < kBins; b += kSampleThreads)
+            bs.masses[b] = joined_mass(massHi[b], rs.massLo[b]);
         __syncthreads();
         span = find_bin(bs, place, span.before, span.massBefore);
         low += (uint64_t) span.bin << shift;
@@ -387,14 +435,13 @@ __device__ inline Candidate locate(const uint64_t *keys, Span span, const Place 
         rs.found = UINT_MAX;
     }
     __syncthreads();
-    for (uint32_t i = t; i < size; i += kSampleThreads) {
-        const uint64_t k = keys[i];
+    each_key<false>(keys, size, [&](uint64_t k) {
         if (k >= low && k <= high) {
             const uint32_t at = atomicAdd(&rs.gathered, 1u);
             if (at < (uint32_t) kRankCap)
                 rs.keys[at] = k;
         }
-    }
+    });
     __syncthreads();
     const uint32_t n = min(rs.gathered, (uint32_t) kRankCap);
     rank_candidates(rs, n);
@@ -423,7 +470,7 @@ __device__ inline Candidate locate(const uint64_t *keys, Span span, const Place 
 // The whole row's state from its chunks' (every thread takes part).
 __device__ inline ChunkState row_state(const ChunkState *chunks, int count)
 {
-    __shared__ double sLargest[kSampleWaves];
+    __shared__ float sLargest[kSampleWaves], sSmallest[kSampleWaves];
     __shared__ int sCount, sLast, sBad, sNans;
     const int t = threadIdx.x;
     if (t == 0) {
@@ -433,10 +480,11 @@ __device__ inline ChunkState row_state(const ChunkState *chunks, int count)
         sNans = 0;
     }
     __syncthreads();
-    double largest = -DBL_MAX;
+    float largest = -INFINITY, smallest = INFINITY;
     for (int i = t; i < count; i += kSampleThreads) {
         const ChunkState c = chunks[i];
-        largest = fmax(largest, c.largest);
+        largest = fmaxf(largest, c.largest);
+        smallest = fminf(smallest, c.smallest);
         atomicAdd(&sCount, c.count);
         atomicMax(&sLast, c.last);
         if (c.bad)
@@ -444,14 +492,20 @@ __device__ inline ChunkState row_state(const ChunkState *chunks, int count)
         if (c.nans)
             atomicAdd(&sNans, c.nans);
     }
-    largest = wave_max_d(largest);
-    if ((t & 63) == 0)
+    largest = max_lanes<32>(largest);
+    smallest = -max_lanes<32>(-smallest);
+    if ((t & 63) == 0) {
         sLargest[t >> 6] = largest;
+        sSmallest[t >> 6] = smallest;
+    }
     __syncthreads();
     ChunkState s{};
-    s.largest = -DBL_MAX;
-    for (int w = 0; w < kSampleWaves; ++w)
-        s.largest = fmax(s.largest, sLargest[w]);
+    s.largest = -INFINITY;
+    s.smallest = INFINITY;
+    for (int w = 0; w < kSampleWaves; ++w) {
+        s.largest = fmaxf(s.largest, sLargest[w]);
+        s.smallest = fminf(s.smallest, sSmallest[w]);
+    }
     s.count = sCount;
     s.last = sLast;
     s.bad = sBad;
@@ -466,7 +520,7 @@ __device__ inline bool masked(const SampleArgs &a, int token)
 
 __global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a, SampleWorkspace w)
 {
-    __shared__ double sLargest[kSampleWaves];
+    __shared__ float sLargest[kSampleWaves], sSmallest[kSampleWaves];
     __shared__ int sCount, sLast, sBad, sNans;
     const int t = threadIdx.x;
     for (int b = blockIdx.x * kSampleThreads + t; b < kBins; b += gridDim.x * kSampleThreads) {
@@ -482,7 +536,6 @@ __global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a
         sNans = 0;
     }
     __syncthreads();
-    const double inverse = 1.0 / (double) a.temperature;
     const int64_t first = (int64_t) blockIdx.x * kChunkTokens + t;
     float logit[kChunkRounds];
     bool live[kChunkRounds];
@@ -492,19 +545,21 @@ __global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a
         live[r] = e < a.vocab && !masked(a, (int) e);
         logit[r] = row_logit(a, e < a.vocab ? e : 0);
     }
-    double largest = -DBL_MAX;
+    float largest = -INFINITY, smallest = INFINITY;
     int count = 0, last = -1, bad = 0, nans = 0;
 #pragma unroll
     for (int r = 0; r < kChunkRounds; ++r)
         if (live[r]) {
-            largest = fmax(largest, candidate_score(logit[r], inverse));
+            largest = fmaxf(largest, logit[r]);
+            smallest = fminf(smallest, logit[r]);
             ++count;
             last = (int) (first + r * kSampleThreads);
             const bool behind = nan_behind(logit[r]);
             nans += behind;
             bad |= !(logit[r] < INFINITY) && !behind;
         }
-    largest = wave_max_d(largest);
+    largest = max_lanes<32>(largest);
+    smallest = -max_lanes<32>(-smallest);
     const double deepest = wave_max_d((double) last); // exact: below 2^31
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1)
@@ -514,6 +569,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a
         atomicAdd(&sNans, nans);
     if ((t & 63) == 0) { // one atomic a wave
         sLargest[t >> 6] = largest;
+        sSmallest[t >> 6] = smallest;
         atomicAdd(&sCount, count);
         atomicMax(&sLast, (int) deepest);
         if (anyBad)
@@ -521,10 +577,11 @@ __global__ __launch_bounds__(kSampleThreads) void sample_max_kernel(SampleArgs a
     }
     __syncthreads();
     if (t == 0) {
-        double m = -DBL_MAX;
-        for (int i = 0; i < kSampleWaves; ++i)
-            m = fmax(m, sLargest[i]);
-        w.chunks[blockIdx.x] = ChunkState{m, 0.0, sCount, sLast, sBad, sNans};
+        for (int i = 1; i < kSampleWaves; ++i) {
+            largest = fmaxf(largest, sLargest[i]);
+            smallest = fminf(smallest, sSmallest[i]);
+        }
+        w.chunks[blockIdx.x] = ChunkState{largest, smallest, 0.0, sCount, sLast, sBad, sNans};
     }
 }
 
@@ -551,16 +608,17 @@ __global__ __launch_bounds__(kSampleThreads) void sample_bins_kernel(SampleArgs 
             sLo[b] = 0ull;
         }
     const ChunkState row = row_state(w.chunks, w.chunkCount); // (syncs)
-    const double inverse = 1.0 / (double) a.temperature, top = row.largest;
+    const double inverse = 1.0 / (double) a.temperature;
+    const BinRule rule = bin_rule(row, inverse, a.vocab);
     double mass = 0.0;
 #pragma unroll
     for (int r = 0; r < kChunkRounds; ++r) {
         if (!live[r])
             continue;
-        const double weight = candidate_weight(logit[r], inverse, top);
+        const double weight = candidate_weight(logit[r], inverse, rule.top);
         mass += weight;
         if (ranked) {
-            const int b = distance_bin(logit[r], inverse, top);
+            const int b = candidate_bin(logit[r], (int) (first + r * kSampleThreads), inverse, rule);
             uint64_t hi = 0, lo = 0;
             if (!row.bad) // else no mass is a number, and none is used
                 split_mass(weight, hi, lo);
@@ -633,7 +691,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_gather_kernel(SampleArg
     const int n = row.count;
     if (n == 0 || !cut(a, n))
         return;
-    const double inverse = 1.0 / (double) a.temperature, top = row.largest;
+    const double inverse = 1.0 / (double) a.temperature;
+    const BinRule rule = bin_rule(row, inverse, a.vocab);
     load_bins(w, sh);
     // the bins' places, and the last bin that the draw reads: the k-th
     // candidate's (whose mass the other searches need), else the one where the
@@ -658,7 +717,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_gather_kernel(SampleArg
     uint32_t place[kChunkRounds];
 #pragma unroll
     for (int r = 0; r < kChunkRounds; ++r) {
-        bin[r] = live[r] ? distance_bin(logit[r], inverse, top) : kBins;
+        bin[r] = live[r] ? candidate_bin(logit[r], (int) (first + r * kSampleThreads), inverse, rule)
+                         : kBins;
         if (bin[r] <= lastBin)
             place[r] = atomicAdd(&sMine[bin[r]], 1u);
     }
@@ -801,7 +861,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(SampleArgs 
     const int t = threadIdx.x;
     const double uniform = a.draws ? a.draws[min(*a.draw_index, a.draw_count - 1)] : a.uniform;
     const ChunkState row = *w.row;
-    const double inverse = 1.0 / (double) a.temperature, top = row.largest;
+    const double inverse = 1.0 / (double) a.temperature, top = top_score(row, inverse);
     const int n = row.count;
     uint32_t chosen = 0;
     if (n > 0 && !cut(a, n)) {

@@ -151,3 +151,27 @@ def test_infinite_temperature_ranks_by_token(torch_cuda, vocab):
                     S(inf, top_p=0.9, seed=63), S(inf, seed=64)):
         got = agree(torch_cuda, row, options, draws=12)
         assert options.top_k != 5 or max(got) < 5
+
+
+@pytest.mark.parametrize("spread", [0.0, 1e-5, 0.01])
+def test_a_crowd_below_an_outlier(torch_cuda, spread):
+    """One token 20 above the rest keeps the bins at their even width, so the
+    rest crowd one or two and the search spreads them again."""
+    vocab = 60000
+    row = np.random.default_rng(12).random(vocab).astype(np.float32) * np.float32(spread)
+    row[777] = 20.0
+    for options in (S(2.0, top_k=2, seed=71), S(4.0, top_k=600, seed=72), S(4.0, top_k=30000, seed=73),
+                    S(4.0, top_p=0.999, seed=74), S(4.0, top_k=50000, top_p=0.9995, seed=75)):
+        agree(torch_cuda, row, options, draws=6)
+
+
+@pytest.mark.parametrize("widest", [1e-44, 1e-30, 0.25, 7.9999995, 8.0, 8.000001, 16.0])
+def test_rows_at_the_edges_of_the_bins_scales(torch_cuda, widest):
+    vocab = 5000
+    row = (-np.random.default_rng(13).random(vocab) * widest).astype(np.float32)
+    row[[100, 4000]] = 0.0, -widest
+    mask = (np.arange(vocab) % 3 == 0).astype(np.float32)
+    mask[[100, 4000]] = 0
+    for options in (S(1.0, top_k=7, seed=81), S(1.0, top_k=3000, seed=82), S(1.0, top_p=0.93, seed=83)):
+        agree(torch_cuda, row, options, draws=4)
+        agree(torch_cuda, row, options, draws=4, mask=mask)

@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <climits>
 
 namespace gq8 {
 namespace {
@@ -908,25 +909,28 @@ __global__ __launch_bounds__(kThreads) void geglu_kernel(const float *__restrict
 }
 
 // Eight outputs a thread (geglu_kernel's values and bytes): the one-output form
-// computes each block's scale 32 times over and stores a byte a lane.  2048
-// rows of 16384: 144 -> 88 us (304 MB, which the copy rate allows in 62).
+// computes each block's scale 32 times over and stores a byte a lane.  Threads
+// run over the pieces of all rows, so a width that is no multiple of a
+// workgroup's leaves none of them idle.  2048 rows of 16384: 144 -> 88 us (304
+// MB, which the copy rate allows in 62).
 __global__ __launch_bounds__(kThreads) void geglu_wide_kernel(const float *__restrict__ fused,
                                                               int rows, int intermediate,
                                                               float *__restrict__ out,
-                                                              uint8_t *__restrict__ q8)
+                                                              uint8_t *__restrict__ q8,
+                                                              uint32_t pieces)
 {
-    const int row = blockIdx.y;
-    const int i = 8 * (blockIdx.x * kThreads + threadIdx.x);
-    if (i >= intermediate) // whole blocks: their four threads leave together
+    const uint32_t piece = blockIdx.x * kThreads + threadIdx.x;
+    if (piece >= pieces) // whole blocks: their four threads leave together
         return;
-    const float *f = fused + (int64_t) row * 2 * intermediate + i;
+    const uint32_t perRow = (uint32_t) intermediate / 8, row = piece / perRow;
+    const float *f = fused + (int64_t) row * 2 * intermediate + 8 * (piece - row * perRow);
     float gate[8], up[8], v[8];
     load_eight(f, gate);
     load_eight(f + intermediate, up);
 #pragma unroll
     for (int k = 0; k < 8; ++k)
         v[k] = geglu(gate[k], up[k]);
-    const int64_t at = (int64_t) row * intermediate + i;
+    const int64_t at = (int64_t) piece * 8;
     if (out)
         store_eight(out + at, v);
     if (q8)
@@ -1031,8 +1035,13 @@ bool aligned_to(const void *p, uintptr_t bytes)
 // The kernels of eight values a thread take over where there are enough values
 // to fill the chip with an eighth of the threads (2048 rows of 2048: quantize
 // 9.3 -> 5.2 us, embed 9.7 -> 6.1); below, more threads with a value each end
-// sooner (geglu of one row of 16384 3.5 against 4.3 us, even at 48 rows).
+// sooner.  The line is where GeGLU to Q8 breaks even (64 rows of 16384 5.9 ->
+// 5.3 us, one row 3.5 -> 4.3); quantize and embed already gain there (4.0 ->
+// 3.1 and 4.2 -> 3.3).  Without Q8 bytes there is no shared work to save, and
+// GeGLU gains by the wider loads alone, later (fp32 only, 64 rows of 16384 4.4
+// against 5.1 us, 256 rows 12.0 against 13.3, 512 rows 20.4 -> 20.0).
 constexpr int64_t kWideElements = 1 << 20;
+constexpr int64_t kWideFloats = 1 << 23;
 
 int argmax_groups(int length)
 {
@@ -1313,10 +1322,11 @@ hipError_t launch_geglu(const float *fused, int rows, int intermediate, float *o
 {
     if (rows <= 0 || intermediate <= 0 || intermediate % kBlock != 0)
         return hipErrorInvalidValue;
-    if ((int64_t) rows * intermediate >= kWideElements && aligned_to(fused, 16)
-        && aligned_to(out, 16) && aligned_to(q8, 8)) {
-        hipLaunchKernelGGL(geglu_wide_kernel, dim3(blocks_for(intermediate, 8 * kThreads), rows),
-                           dim3(kThreads), 0, stream, fused, rows, intermediate, out, q8);
+    const int64_t elements = (int64_t) rows * intermediate, pieces = elements / 8;
+    if (elements >= (q8 ? kWideElements : kWideFloats) && rows <= 65535 && pieces <= INT_MAX
+        && aligned_to(fused, 16) && aligned_to(out, 16) && aligned_to(q8, 8)) {
+        hipLaunchKernelGGL(geglu_wide_kernel, dim3(blocks_for(pieces, kThreads)), dim3(kThreads), 0,
+                           stream, fused, rows, intermediate, out, q8, (uint32_t) pieces);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(geglu_kernel, dim3(blocks_for(intermediate, kThreads), rows),

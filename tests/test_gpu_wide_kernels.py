@@ -78,3 +78,22 @@ def test_embed_wide(torch_cuda, rows, width):
         G.embed(idd.data_ptr() + 4 * r, 1, td.data_ptr(), vocab, width, 45.254833, one.data_ptr())
         torch.cuda.synchronize()
         assert torch.equal(out[r], one[0])
+
+
+@pytest.mark.parametrize("rows,inter", [(32770, 32), (4099, 256), (1011, 2080)])
+def test_geglu_wide_rows_that_share_workgroups(torch_cuda, rows, inter):
+    """Rows narrower than a workgroup's values, or not a multiple of them."""
+    test_geglu_wide(torch_cuda, rows, inter)
+
+
+def test_geglu_wide_floats_alone(torch_cuda):
+    """fp32 values without Q8 bytes change over at eight million."""
+    torch = torch_cuda
+    rows, inter = 513, 16384
+    fused = torch.randn(rows, 2 * inter, device="cuda")
+    out, one = torch.empty(rows, inter, device="cuda"), torch.empty(1, inter, device="cuda")
+    G.geglu(fused.data_ptr(), rows, inter, out.data_ptr(), None)
+    for r in (0, 1, rows // 2, rows - 1):
+        G.geglu(fused[r].data_ptr(), 1, inter, one.data_ptr(), None)
+        torch.cuda.synchronize()
+        assert torch.equal(out[r], one[0])

@@ -429,39 +429,48 @@ hipError_t launch_tile(const TileArgs &a, hipStream_t stream)
 // is at most one workgroup a compute unit takes `alone` microseconds per 2048
 // of the inner size (a workgroup's chain of chunks); n workgroups a compute
 // unit take n times `packed` (n rounded up: the fullest unit ends last).
-// Both were fitted to a sweep on one MI355X over rows 2 .. 2048, inner sizes
-// 2048 and 16384 and 512 .. 256000 outputs, weights from HBM; the estimate
-// was within 10 % of most points and its choice within 15 % of the fastest
-// tile.  Microseconds there, the 128 x 64 tile (the only one before) -> the
-// chosen one: 16384 -> 2048 at 64 rows 165 -> 25, at 512 169 -> 90, at 1024
-// 171 -> 154; 2048 -> 2048 at 64 rows 22.9 -> 5.8, at 512 24.5 -> 15.9; 2048
-// -> 32768 at 32 rows 39 -> 19.5, at 64 40 -> 25 (at 128 and more it stays).
-// Below 32 rows, where the products had run in q8_product_kernel: 2048 ->
-// 32768 at 16 rows 80 -> 15.4 (4.7 TB/s of weights), 16384 -> 2048 70 -> 19.5,
-// 2048 -> 256000 at 5 rows 324 -> 92 (6.1 TB/s).
+// Below an inner size of kShortInner a workgroup's staging, merge and store
+// weigh as much as its chain, and `start` microseconds a round come on top of
+// it (256 -> 1024 at 1500 rows: 10.3 us by the chains alone, 6.5 so; 77 of the
+// 126 points at 256 and 512 gained, by 1.2 us, and none lost).
+// All were fitted to sweeps on one MI355X over rows 2 .. 2048, inner sizes 256
+// .. 16384 and 256 .. 256000 outputs, weights from HBM.  The estimate ranks the
+// tiles and is no time: what every launch costs (2.5 to 5 us) is left out, so
+// it is within 10 % at 35 of 59 points at an inner size of 16384 and 0.64 of
+// the time in the median at 2048.  The choice is within 10 % of the fastest
+// tile at nine points of ten and within 15 % at 421 of 434; the worst is
+// 16384 -> 8192 at 17 rows, 51 against 38 us.  Microseconds, the 128 x 64 tile
+// (the only one before) -> the chosen one: 16384 -> 2048 at 64 rows 165 -> 25,
+// at 512 169 -> 90, at 1024 171 -> 154; 2048 -> 2048 at 64 rows 22.9 -> 5.8, at
+// 512 24.5 -> 15.9; 2048 -> 32768 at 32 rows 39 -> 19.5, at 64 40 -> 25 (at 128
+// and more it stays).  Below 32 rows, where the products had run in
+// q8_product_kernel: 2048 -> 32768 at 16 rows 80 -> 15.4 (4.7 TB/s of weights),
+// 16384 -> 2048 70 -> 19.5, 2048 -> 256000 at 5 rows 324 -> 92 (6.1 TB/s).
 struct TileCost {
     int rows, outputs; // the tile
     double alone, packed;
     hipError_t (*launch)(const TileArgs &, hipStream_t);
+    double start; // below kShortInner
 };
 
+constexpr int kShortInner = 1024;
 constexpr int kComputeUnits = 256;
 constexpr int kMaxTileRows = 65535; // the grid's y extent
 
 const TileCost kProductTiles[] = {
-    {128, 64, 20.2, 18.2, launch_tile<Tile128x64, false, false>},
-    {64, 64, 11.3, 10.0, launch_tile<Tile64x64, false, true>},
-    {64, 32, 6.6, 5.6, launch_tile<Tile64x32, false, true>},
-    {32, 64, 6.8, 6.4, launch_tile<Tile32x64, false, true>},
-    {16, 32, 3.6, 2.3, launch_tile<Tile16x32, false, true>},
-    {32, 16, 2.7, 2.7, launch_tile<Tile32x16, false, true>},
-    {16, 16, 2.1, 1.5, launch_tile<Tile16x16, false, true>},
+    {128, 64, 20.2, 18.2, launch_tile<Tile128x64, false, false>, 0.2},
+    {64, 64, 11.3, 10.0, launch_tile<Tile64x64, false, true>, 0.5},
+    {64, 32, 6.6, 5.6, launch_tile<Tile64x32, false, true>, 0.4},
+    {32, 64, 6.8, 6.4, launch_tile<Tile32x64, false, true>, 0.4},
+    {16, 32, 3.6, 2.3, launch_tile<Tile16x32, false, true>, 0.2},
+    {32, 16, 2.7, 2.7, launch_tile<Tile32x16, false, true>, 3.0},
+    {16, 16, 2.1, 1.5, launch_tile<Tile16x16, false, true>, 0.4},
 };
 const TileCost kGegluTiles[] = { // 64 staged weight rows: 32 outputs
-    {128, 64, 20.2, 18.2, launch_tile<Tile128x64, true, false>},
-    {64, 64, 11.3, 10.0, launch_tile<Tile64x64, true, true>},
-    {32, 64, 6.8, 6.4, launch_tile<Tile32x64, true, true>},
-    {16, 64, 5.4, 4.7, launch_tile<Tile16x64, true, true>},
+    {128, 64, 20.2, 18.2, launch_tile<Tile128x64, true, false>, 0.0},
+    {64, 64, 11.3, 10.0, launch_tile<Tile64x64, true, true>, 0.0},
+    {32, 64, 6.8, 6.4, launch_tile<Tile32x64, true, true>, 0.0},
+    {16, 64, 5.4, 4.7, launch_tile<Tile16x64, true, true>, 0.0},
 };
 
 template <size_t N>
@@ -477,7 +486,8 @@ hipError_t launch_best(const TileCost (&tiles)[N], const TileArgs &a, hipStream_
             continue;
         const int64_t workgroups = tileRows * ((a.outputs + (int64_t) c.outputs - 1) / c.outputs);
         const int64_t rounds = (workgroups + kComputeUnits - 1) / kComputeUnits;
-        const double cost = std::max(c.alone, (double) rounds * c.packed);
+        const double chain = a.inner / 2048.0 * std::max(c.alone, (double) rounds * c.packed);
+        const double cost = chain + (a.inner < kShortInner ? (double) rounds * c.start : 0.0);
         if (!best || cost < least) {
             best = &c;
             least = cost;

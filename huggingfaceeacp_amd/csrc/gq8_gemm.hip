@@ -474,29 +474,41 @@ const TileCost kGegluTiles[] = { // 64 staged weight rows: 32 outputs
 };
 
 template <size_t N>
-hipError_t launch_best(const TileCost (&tiles)[N], const TileArgs &a, hipStream_t stream)
+const TileCost &best_tile(const TileCost (&tiles)[N], int rows, int inner, int outputs)
 {
     const TileCost *best = nullptr;
     double least = 0.0;
     for (const TileCost &c : tiles) {
-        if (c.rows == 128 && a.inner % (Tile128x64::chunk * kBlock) != 0)
+        if (c.rows == 128 && inner % (Tile128x64::chunk * kBlock) != 0)
             continue; // the large tile takes whole chunks
-        const int64_t tileRows = (a.rows + (int64_t) c.rows - 1) / c.rows;
+        const int64_t tileRows = (rows + (int64_t) c.rows - 1) / c.rows;
         if (tileRows > kMaxTileRows && c.rows < 64)
             continue;
-        const int64_t workgroups = tileRows * ((a.outputs + (int64_t) c.outputs - 1) / c.outputs);
+        const int64_t workgroups = tileRows * ((outputs + (int64_t) c.outputs - 1) / c.outputs);
         const int64_t rounds = (workgroups + kComputeUnits - 1) / kComputeUnits;
-        const double chain = a.inner / 2048.0 * std::max(c.alone, (double) rounds * c.packed);
-        const double cost = chain + (a.inner < kShortInner ? (double) rounds * c.start : 0.0);
+        const double chain = inner / 2048.0 * std::max(c.alone, (double) rounds * c.packed);
+        const double cost = chain + (inner < kShortInner ? (double) rounds * c.start : 0.0);
         if (!best || cost < least) {
             best = &c;
             least = cost;
         }
     }
-    return best->launch(a, stream);
+    return *best;
+}
+
+template <size_t N>
+hipError_t launch_best(const TileCost (&tiles)[N], const TileArgs &a, hipStream_t stream)
+{
+    return best_tile(tiles, a.rows, a.inner, a.outputs).launch(a, stream);
 }
 
 } // namespace
+
+ProductTile q8_gemm_tile(int rows, int inner, int outputs)
+{
+    const TileCost &c = best_tile(kProductTiles, rows, inner, outputs);
+    return {c.rows, c.outputs};
+}
 
 hipError_t launch_q8_gemm(const uint8_t *x8, int64_t x_elements, int x_row0, int rows,
                           const uint8_t *w8, int inner, int outputs, float *y, int y_stride,

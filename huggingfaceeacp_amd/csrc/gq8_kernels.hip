@@ -1219,48 +1219,56 @@ hipError_t launch_matvec(const uint8_t *x8, int64_t xElements, int xRow, const u
 }
 
 constexpr size_t kProductLdsLimit = 64 * 1024;
+constexpr int kMaxInner = 16384; // of every product
 
 size_t product_lds(int b, int inner)
 {
     return (size_t) b * inner + (size_t) b * (inner / kBlock) * sizeof(double);
 }
+
+// Whether waves take whole weight rows.  One row: always, but for a
+// vocabulary-wide product of a weight row a wave reads at once, which the 16 x
+// 32 MFMA tile streams faster (256 -> 131072 18.9 -> 15.1 us, 512 -> 262144
+// 39.3 -> 32.9, 1024 -> 131072 27.0 -> 27.8, 2048 -> 256000 95 -> 89).
+// A few rows: in a narrow product, whose weights they stream better than the
+// tiles do (2 rows of 16384 -> 2048: 14.1 against 19.5 us, of 2048 -> 2048: 4.0
+// against 4.9; 4 rows 4.7 against 5.0; at 5 the tiles lead, 5.5 against 5.0).
+// A wide one (2 rows of 2048 -> 32768: 17.3 against 15.0) is the tiles'.  The
+// line leaves some of the tiles' gains near its ends: 8192 outputs (4 rows of
+// 2048 8.9 against 6.8, 2 rows of 16384 35.9 against 29.7), and four rows that
+// do not fit LDS and go two at a time (16384 -> 2048: 21.3 against 19.7).
+bool whole_weight_rows(int rows, int inner, int outputs)
+{
+    if (rows == 1)
+        return outputs < 131072 || inner > 2048;
+    return rows <= 4 && outputs < 16384;
+}
 } // namespace
+
+ProductTile q8_product_tile(int rows, int inner, int outputs)
+{
+    return whole_weight_rows(rows, inner, outputs) ? ProductTile{0, 0}
+                                                   : q8_gemm_tile(rows, inner, outputs);
+}
 
 hipError_t launch_q8_product(const uint8_t *x8, int x_rows_total, int x_row0, int rows,
                              const uint8_t *w8, int inner, int outputs, float *y, int y_stride,
                              int residual, hipStream_t stream)
 {
     if (rows <= 0 || inner <= 0 || outputs <= 0 || inner % kBlock != 0 || y_stride < outputs
-        || x_row0 < 0 || x_row0 + rows > x_rows_total || product_lds(1, inner) > kProductLdsLimit)
+        || x_row0 < 0 || x_row0 + rows > x_rows_total || inner > kMaxInner)
         return hipErrorInvalidValue;
     const int64_t xElements = (int64_t) x_rows_total * inner;
-    // one row: whole weight rows a wave, but for a vocabulary-wide product, which
-    // the 16 x 32 MFMA tile streams faster (2048 -> 256000: 94 against 87 us)
-    if (rows == 1 && (outputs < 131072 || inner > 2048))
+    if (!whole_weight_rows(rows, inner, outputs))
+        return launch_q8_gemm(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride, residual,
+                              stream);
+    if (rows == 1)
         return launch_matvec(x8, xElements, x_row0, w8, inner, outputs, y, residual, stream);
-    // a few rows of a narrow product: whole weight rows a wave stream better
-    // than the MFMA tiles do (2 rows of 16384 -> 2048: 13.4 against 19.3 us,
-    // of 2048 -> 2048: 4.0 against 4.6; even at 4 rows, 21.2 and 4.2 against
-    // 19.4 and 4.6; at 5 the tiles lead, 27 and 5.5 against 19.5 and 4.6).  A
-    // wide one (2 rows of 2048 -> 32768: 17.3 against 15.0) is the tiles'.
-    if (rows <= 4 && outputs < 16384) {
-        int b = 4;
-        while (b > 1 && (b > rows || product_lds(b, inner) > kProductLdsLimit))
-            b >>= 1;
-        switch (b) {
-        case 4:
-            return product_with<4>(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride,
-                                   residual, stream);
-        case 2:
-            return product_with<2>(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride,
-                                   residual, stream);
-        default:
-            return product_with<1>(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride,
-                                   residual, stream);
-        }
-    }
-    return launch_q8_gemm(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride, residual,
-                          stream);
+    if (rows == 4 && product_lds(4, inner) <= kProductLdsLimit)
+        return product_with<4>(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride, residual,
+                               stream);
+    return product_with<2>(x8, xElements, x_row0, rows, w8, inner, outputs, y, y_stride, residual,
+                           stream);
 }
 
 size_t mqa_workspace_bytes(int rows, int heads, int head_dim, int max_keys)

@@ -57,6 +57,13 @@ bool q8_gemm_geglu_supported(int rows, int inner, int intermediate);
 hipError_t launch_q8_gemm_geglu(const uint8_t *x8, int64_t x_elements, int x_row0, int rows,
                                 const uint8_t *w8, int inner, int intermediate, uint8_t *q8_out,
                                 float *debug_out, hipStream_t stream);
+// The tile of y that a workgroup of the product takes; 0 x 0 where waves take
+// whole weight rows.
+struct ProductTile {
+    int rows, outputs;
+};
+ProductTile q8_product_tile(int rows, int inner, int outputs);
+ProductTile q8_gemm_tile(int rows, int inner, int outputs);
 hipError_t launch_q8_gemm(const uint8_t *x8, int64_t x_elements, int x_row0, int rows,
                           const uint8_t *w8, int inner, int outputs, float *y, int y_stride,
                           int residual, hipStream_t stream);

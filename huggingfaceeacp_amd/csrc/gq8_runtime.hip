@@ -321,6 +321,18 @@ extern "C" int gq8_q8_product(const uint8_t *x8, const uint8_t *w8, int rows, in
     return GQ8_OK;
 }
 
+extern "C" int gq8_q8_product_tile(int rows, int inner, int outputs, int *tile_rows,
+                                   int *tile_outputs)
+{
+    if (rows <= 0 || inner <= 0 || outputs <= 0 || inner % gq8::kBlock != 0 || inner > 16384
+        || !tile_rows || !tile_outputs)
+        return fail(GQ8_ERR_ARGUMENT, "q8_product_tile: bad arguments");
+    const gq8::ProductTile tile = gq8::q8_product_tile(rows, inner, outputs);
+    *tile_rows = tile.rows;
+    *tile_outputs = tile.outputs;
+    return GQ8_OK;
+}
+
 extern "C" int gq8_kv_store_f16(const float *k, const float *v, int src_stride, int rows,
                                 int kv_width, uint16_t *key_cache, uint16_t *value_cache,
                                 int position, void *stream)

@@ -122,6 +122,7 @@ def library() -> ctypes.CDLL:
         "gq8_rmsnorm": (i32, [P, P, i32, i32, f32, P, P, P]),
         "gq8_rope": (i32, [P, i32, i32, i32, i32, i32, P, P, P]),
         "gq8_q8_product": (i32, [P, P, i32, i32, i32, P, i32, i32, P]),
+        "gq8_q8_product_tile": (i32, [i32, i32, i32, P, P]),
         "gq8_kv_store_f16": (i32, [P, P, i32, i32, i32, P, P, i32, P]),
         "gq8_mqa_workspace_bytes": (sz, [i32, i32, i32, i32]),
         "gq8_mqa_decode": (i32, [P, P, P, i32, i32, i32, i32, f32, P, P, sz, P]),
@@ -266,6 +267,15 @@ def rope(x, row_stride, heads, head_dim, first_position, rows, cosines, sines, s
 def q8_product(x8, w8, rows, inner, outputs, y, y_stride, residual=False, stream=0):
     return check(library().gq8_q8_product(x8, w8, rows, inner, outputs, y, y_stride,
                                           int(residual), stream))
+
+
+def q8_product_tile(rows, inner, outputs):
+    """(rows, outputs) of the tile a workgroup of q8_product takes; (0, 0) where
+    waves take whole weight rows."""
+    tile = (ctypes.c_int * 2)()
+    check(library().gq8_q8_product_tile(rows, inner, outputs, ctypes.byref(tile),
+                                        ctypes.addressof(tile) + ctypes.sizeof(ctypes.c_int)))
+    return tuple(tile)
 
 
 def kv_store_f16(k, v, src_stride, rows, kv_width, key_cache, value_cache, position, stream=0):

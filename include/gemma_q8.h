@@ -109,6 +109,11 @@ int gq8_rope(float *x, int row_stride, int heads, int head_dim, int first_positi
 int gq8_q8_product(const uint8_t *x8, const uint8_t *w8, int rows, int inner, int outputs,
                    float *y, int y_stride, int residual, void *stream);
 
+/* The tile of y (rows x outputs) that one workgroup of gq8_q8_product takes for
+ * these sizes, 0 x 0 where single waves take whole weight rows.  Host
+ * arithmetic alone. */
+int gq8_q8_product_tile(int rows, int inner, int outputs, int *tile_rows, int *tile_outputs);
+
 /* fp16 KV-cache append (the ranged bind of Decoder.cpp:450-466, with fp16
  * storage): rows of k and v (fp32, row stride src_stride) written at cache
  * rows position .. position + rows - 1 of [max_positions, kv_width] caches. */

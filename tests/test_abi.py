@@ -61,6 +61,24 @@ def test_algorithmic_decode_bytes_closed_form():
             2_662_727_680 + 303_104 + 2_176 + 18_432 * L + 18_432)
 
 
+@pytest.mark.parametrize("rows,inner,outputs,tile", [
+    (1, 2048, 255968, (16, 32)), (1, 2048, 131071, (0, 0)), (1, 4096, 256000, (0, 0)),
+    (2, 16384, 2048, (0, 0)), (4, 2048, 16383, (0, 0)), (4, 2048, 16384, (16, 32)),
+    (5, 16384, 2048, (16, 16)), (24, 2048, 32768, (32, 64)), (512, 16384, 2048, (64, 32)),
+    (2048, 2048, 32768, (128, 64)), (2048, 2080, 32768, (64, 64)),
+    # a short inner size: few rounds of workgroups, not few chunks
+    (1500, 256, 1024, (128, 64)), (2048, 64, 1000, (64, 64))])
+def test_product_tile_choice(rows, inner, outputs, tile):
+    assert G.q8_product_tile(rows, inner, outputs) == tile
+
+
+@pytest.mark.parametrize("bad", [(0, 32, 1), (1, 48, 1), (1, 16416, 1), (1, 32, 0)])
+def test_product_tile_refusals(bad):
+    with pytest.raises(G.Gq8Error) as info:
+        G.q8_product_tile(*bad)
+    assert info.value.status == G.ERR_ARGUMENT
+
+
 def test_host_quantizer_matches_the_oracle():
     rng = np.random.default_rng(5)
     values = np.concatenate([rng.standard_normal(1 << 16).astype(np.float32) * 0.02,

@@ -210,13 +210,17 @@ def test_q8_product_rows_and_residual(torch_cuda, rows):
 
 @pytest.mark.parametrize("rows,inner,outputs", [(32, 2048, 2560), (64, 2048, 2048),
                                                  (100, 16384, 2048), (130, 64, 96),
-                                                 (33, 2048, 32768), (300, 512, 200)])
+                                                 (33, 2048, 32768), (300, 512, 200),
+                                                 (97, 256, 8210), (65, 768, 12290)])
 def test_q8_gemm_rows_are_the_one_row_products(torch_cuda, rows, inner, outputs):
-    """Steps of 32 rows or more run on the int8 MFMA GEMM (an inner size of
-    64 takes the row kernel); each row is the exact block dot scaled and
-    summed in double in block order, as the oracle does, so the rows are
-    bit-identical to the one-row products.  Shapes cover whole and partial
-    128 x 64 tiles and one to 64 K chunks."""
+    """Steps of several rows run on the int8 MFMA GEMM; each row is the exact
+    block dots scaled and summed in double.  The 128 x 64 tile (the last two
+    shapes) adds them in block order, as the oracle does, so its rows are
+    bit-identical to the one-row products; the other tiles' waves take a
+    chunk's blocks apart and add their sums at the end, a few 2^-53 off, and
+    with these inputs every fp32 they round to is the same."""
+    if (rows, inner, outputs) in ((97, 256, 8210), (65, 768, 12290)):
+        assert G.q8_product_tile(rows, inner, outputs) == (128, 64)
     torch = torch_cuda
     w = O.quantize_int8_blocks(spread(inner * outputs, 81, 0.02))
     x = spread(rows * inner, 82, 1.0)

@@ -11,27 +11,32 @@ from huggingfaceeacp_amd import gemma_q8 as G
 
 pytestmark = pytest.mark.gpu
 
-# (rows, outputs): the tile the choice takes for them
-TILES = {
-    "whole rows a wave": (4, 70),
-    "16 x 16": (17, 34),
-    "16 x 16, two rounds": (33, 2050),
-    "32 x 16": (60, 2040),
-    "16 x 32": (35, 8210),
-    "32 x 64": (31, 9002),
-    "64 x 32": (130, 2046),
-    "64 x 64": (257, 2090),
-    "128 x 64": (2040, 2046),
-}
+# (tile, rows, outputs, inner sizes): rows and outputs that are no multiples of
+# the tile; (0, 0) is whole weight rows a wave
+TILES = [
+    ((0, 0), 4, 70, (32, 96, 256, 1056, 1280)),
+    ((0, 0), 3, 2046, (96, 1056, 16384)),
+    ((16, 16), 17, 34, (768, 1056, 1280)),
+    ((16, 16), 33, 2050, (1056, 1280)),         # two rounds of workgroups
+    ((16, 32), 17, 34, (32, 96, 256)),
+    ((16, 32), 35, 8210, (768, 1056, 1280)),
+    ((32, 16), 60, 2040, (1056, 1280)),
+    ((32, 64), 31, 9002, (32, 96, 256, 1056, 1280)),
+    ((64, 32), 130, 2046, (32, 96, 256, 1056, 1280)),
+    ((64, 64), 33, 8210, (32, 96, 256)),
+    ((64, 64), 257, 2090, (768,)),
+    ((64, 64), 97, 12290, (1056,)),
+    ((64, 64), 2040, 2046, (32, 96)),
+    ((128, 64), 97, 8210, (256,)),
+    ((128, 64), 2040, 2046, (256, 768)),
+]
 
 
-@pytest.mark.parametrize("inner", [32, 96, 256, 1056, 1280])
-@pytest.mark.parametrize("tile", list(TILES))
-def test_product_tile_edges(torch_cuda, tile, inner):
+@pytest.mark.parametrize("tile,rows,outputs,inner", [
+    (tile, rows, outputs, inner) for tile, rows, outputs, inners in TILES for inner in inners])
+def test_product_tile_edges(torch_cuda, tile, rows, outputs, inner):
     torch = torch_cuda
-    rows, outputs = TILES[tile]
-    if inner > 256 and rows * outputs > 1 << 20:
-        inner = 768  # the oracle's time; still whole and several chunks
+    assert G.q8_product_tile(rows, inner, outputs) == tile
     nb, stride = inner // 32, outputs + 3
     w = O.quantize_int8_blocks(spread(inner * outputs, 91, 0.05))
     q, s = O.quantize_row(spread(rows * inner, 92, 1.0))

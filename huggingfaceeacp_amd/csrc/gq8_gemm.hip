@@ -7,9 +7,12 @@
 // SimdTiledMatMul.h / TiledMatMul.h) with both operands in Int8Blocks: the
 // activation rows quantized by the reference's own weight rule.  One
 // v_mfma_i32_16x16x32_i8 covers exactly one block of a 16 x 16 tile, so every
-// block's integer dot is exact; it is then scaled and accumulated in double,
-// block by block in order, exactly as the one-row kernels and the oracle do
-// -- so a prompt row computed here equals the same row computed alone.
+// block's integer dot is exact; it is then scaled and accumulated in double.
+// The 128 x 64 tile adds a row's blocks in order, as the oracle does.  The
+// others' waves take the blocks of a chunk apart (KS) and add their sums at
+// the end, so the order of a row's sum depends on the tile, and with it on how
+// many rows share the step: equal to the row computed alone but for a few
+// 2^-53 before the result is rounded to fp32, which is rarely seen in it.
 //
 // Tiling (TileShape): a workgroup of eight waves owns a TM x TN tile of y
 // (rows x outputs), a wave RM x RN MFMA tiles of it over 1 / KS of every

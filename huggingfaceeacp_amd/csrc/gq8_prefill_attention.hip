@@ -13,7 +13,7 @@
 // head).  Fewer than 16 rows take one row a block, so no row's arithmetic
 // meets another row's keys.  The block's key tiles (16 keys) are split over
 // several workgroups where the blocks alone would leave the chip idle or end
-// unevenly (split_plan); a workgroup's four waves take its tiles round robin,
+// unevenly (attention_split); a workgroup's four waves take its tiles round robin,
 // each keeping an online softmax state (row maximum, sum and the 16 x head_dim
 // sums), and the states are merged in LDS at the end.  A block in one
 // workgroup finishes its rows there; the splits of one leave their scaled sums,
@@ -410,6 +410,12 @@ bool tiled_attention_supported(int head_dim, const float *queries, int q_stride,
 // rows behind 700 keys 99 -> 77, 128 behind 4000 352 -> 105, 16 behind 8000
 // 672 -> 42, one row of 8000 keys 680 -> 27 (110 in mqa_partial_kernel and its
 // former merge); 512 rows behind 512 keys and 2048 alone stay whole (94, 330).
+// The same constants serve narrower heads, whose rounds are shorter but whose
+// workgroups do overlap on a unit: 2 to 4 times faster than whole blocks over
+// long caches (512 rows behind 4000 keys at 4 heads of 64 131 -> 67), and up
+// to 17 % slower where some 100 keys are split after all (64 rows behind 100
+// keys at 16 heads of 64 9.4 -> 11.0).  Rounds scaled by the head width keep
+// those whole, but lose 5 to 30 % at thirty other points of the sweep.
 AttentionSplit attention_split(int rows, int heads, int kv_heads, int keys)
 {
     constexpr int kUnits = 256, kSamples = 32;

@@ -122,7 +122,9 @@ int gq8_kv_store_f16(const float *k, const float *v, int src_stride, int rows, i
 
 /* MultiQueryDecodeAttention (MultiQueryAttention.h:317-341): one query row of
  * heads x head_dim over key_count fp16 cached rows, split over key chunks with
- * an exact online-softmax merge.  workspace >= gq8_mqa_workspace_bytes(). */
+ * an exact online-softmax merge.  workspace >= gq8_mqa_workspace_bytes(): it
+ * holds the splits until the stream has run the call, so calls that may run
+ * at the same time (two streams) take one each. */
 size_t gq8_mqa_workspace_bytes(int rows, int heads, int head_dim, int max_keys);
 int gq8_mqa_decode(const float *query, const uint16_t *key_cache, const uint16_t *value_cache,
                    int heads, int kv_heads, int head_dim, int key_count, float scale, float *out,
@@ -145,7 +147,8 @@ int gq8_mqa_decode_noalloc(const float *query, const uint16_t *key_cache,
                            int key_count, float scale, float *out, void *stream);
 
 /* MultiQueryPrefillAttention (MultiQueryAttention.h:275-308): rows query rows
- * at positions position_offset + r, row r over keys [0, position_offset + r]. */
+ * at positions position_offset + r, row r over keys [0, position_offset + r].
+ * The workspace as gq8_mqa_decode's, for any row count. */
 int gq8_mqa_prefill(const float *queries, const uint16_t *key_cache,
                     const uint16_t *value_cache, int heads, int kv_heads, int head_dim,
                     int rows, int position_offset, float scale, float *out, void *workspace,
@@ -439,7 +442,8 @@ int gq8_batch_prefill(gq8_batch *batch, int sequence, const int32_t *prompt, int
  * writes its argmax into the next slot and advances the position (the
  * greedy loop's step, Gemma.cpp:320-333, for every sequence at once); no EOS
  * check.  GQ8_ERR_NOT_PREPARED if a sequence has no prompt, GQ8_ERR_WINDOW if
- * one would pass max_positions.  use_graph != 0 replays one captured step.
+ * one would pass max_positions.  use_graph != 0 replays a captured step (one a
+ * range of the longest row's keys, captured before the run's first step).
  * Synchronous. */
 int gq8_batch_decode(gq8_batch *batch, int steps, int use_graph);
 int gq8_batch_sequences(const gq8_batch *batch);

@@ -68,6 +68,23 @@ struct ChunkState {
     int nans;       // NaNs with the sign set, which rank after every number
 };
 
+// The bins of a row.  A score lies `distance` = top - score below the largest:
+// 64 bins a unit up to 16, then 64 an octave (the top bits of the distance as
+// a float), the last one for all that lie past 2^20.  Where all scores lie
+// within 8 of the largest, distances are scaled by a power of two to fill the
+// even bins, and where they tie, the bins go by token (`tokens` each): a flat
+// row's candidates do not crowd a few bins.
+struct BinRule {
+    double top, scale; // bins a unit of distance
+    int tokens;        // 0: by distance
+};
+
+// The whole row: its chunks together, and its bins.
+struct RowState {
+    ChunkState all;
+    BinRule rule;
+};
+
 // What the gather leaves for the draw.
 struct Gathered {
     double total; // the row's mass
@@ -77,7 +94,7 @@ struct Gathered {
 
 struct SampleWorkspace {
     ChunkState *chunks;
-    ChunkState *row;    // the whole row's
+    RowState *row;
     Gathered *summary;
     uint32_t *counts;   // of the bins
     uint32_t *cursors;  // candidates of a bin gathered so far
@@ -146,25 +163,14 @@ __device__ inline bool nan_behind(float logit)
     return logit != logit && (__float_as_uint(logit) >> 31);
 }
 
-// The bins of a row.  A score lies `distance` = top - score below the largest:
-// 64 bins a unit up to 16, then 64 an octave (the top bits of the distance as
-// a float), the last one for all that lie past 2^20.  Where all scores lie
-// within 8 of the largest, distances are scaled by a power of two to fill the
-// even bins, and where they tie, the bins go by token (`tokens` each): a flat
-// row's candidates do not crowd a few bins.
-struct BinRule {
-    double top, scale;
-    int tokens; // 0: by distance
-};
-
 __device__ inline BinRule bin_rule(const ChunkState &row, double inverse, int vocab)
 {
-    BinRule rule{top_score(row, inverse), 1.0, 0};
+    BinRule rule{top_score(row, inverse), 64.0, 0};
     const double range = rule.top - candidate_score(row.smallest, inverse);
     if (range == 0.0)
         rule.tokens = (vocab + kBins - 1) / kBins;
     else if (range > 0.0 && range < 8.0)
-        rule.scale = ldexp(1.0, min(3 - ilogb(range), 1000));
+        rule.scale = ldexp(64.0, min(3 - ilogb(range), 1000));
     return rule;
 }
 
@@ -173,15 +179,15 @@ __device__ inline BinRule bin_rule(const ChunkState &row, double inverse, int vo
 // distance to itself is a NaN of clear sign).
 __device__ inline int candidate_bin(float logit, int token, double inverse, const BinRule &rule)
 {
-    const double distance = (rule.top - candidate_score(logit, inverse)) * rule.scale;
-    if (!(distance >= 0.0))
+    const double steps = (rule.top - candidate_score(logit, inverse)) * rule.scale;
+    if (!(steps >= 0.0))
         return nan_behind(logit) ? kBins - 1 : 0;
     if (rule.tokens)
         return token / rule.tokens;
-    if (distance < 16.0)
-        return (int) (distance * 64.0);
-    const float f = (float) fmin(distance, 1e30);
-    const int octaves = (int) (__float_as_uint(f) >> 17) - (int) (__float_as_uint(16.f) >> 17);
+    if (steps < kBins / 2)
+        return (int) steps;
+    const float f = (float) fmin(steps, 1e30);
+    const int octaves = (int) (__float_as_uint(f) >> 17) - (int) (__float_as_uint(kBins / 2) >> 17);
     return min(kBins / 2 + octaves, kBins - 1);
 }
 
@@ -635,7 +641,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_bins_kernel(SampleArgs 
     if (t == 0) {
         w.chunks[blockIdx.x].mass = mt;
         if (blockIdx.x == 0)
-            *w.row = row;
+            *w.row = RowState{row, rule};
     }
     if (ranked)
         for (int b = t; b < kBins; b += kSampleThreads)
@@ -687,12 +693,12 @@ __global__ __launch_bounds__(kSampleThreads) void sample_gather_kernel(SampleArg
         live[r] = e < a.vocab && !masked(a, (int) e);
         logit[r] = row_logit(a, e < a.vocab ? e : 0);
     }
-    const ChunkState row = *w.row;
+    const ChunkState row = w.row->all;
+    const BinRule rule = w.row->rule;
     const int n = row.count;
     if (n == 0 || !cut(a, n))
         return;
     const double inverse = 1.0 / (double) a.temperature;
-    const BinRule rule = bin_rule(row, inverse, a.vocab);
     load_bins(w, sh);
     // the bins' places, and the last bin that the draw reads: the k-th
     // candidate's (whose mass the other searches need), else the one where the
@@ -860,8 +866,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(SampleArgs 
     __shared__ RankShared ranks;
     const int t = threadIdx.x;
     const double uniform = a.draws ? a.draws[min(*a.draw_index, a.draw_count - 1)] : a.uniform;
-    const ChunkState row = *w.row;
-    const double inverse = 1.0 / (double) a.temperature, top = top_score(row, inverse);
+    const ChunkState row = w.row->all;
+    const double inverse = 1.0 / (double) a.temperature, top = w.row->rule.top;
     const int n = row.count;
     uint32_t chosen = 0;
     if (n > 0 && !cut(a, n)) {
@@ -875,53 +881,45 @@ __global__ __launch_bounds__(kSampleThreads) void sample_draw_kernel(SampleArgs 
         uint32_t cb, ct;
         double mb, all;
         workgroup_scan(0u, bins.masses[2 * t] + bins.masses[2 * t + 1], cb, mb, ct, all, bins.scan);
-        // the bin of a place, and the candidate in it (its bin's gathered
-        // candidates; `locate` may use the bins' space, which is then loaded
-        // again)
-        auto find_in = [&](const Span &span, const Place &place) {
-            const Candidate c = locate(w.gathered + span.before, span, place, inverse, top, bins, ranks);
-            if (span.count > (uint32_t) kRankCap)
-                load_bins(w, bins);
-            return c;
-        };
-        auto find = [&](const Place &place) { return find_in(find_bin(bins, place, 0u, 0.0), place); };
         int kept = first_kept(a, n);
         const bool sums = weights_are_numbers(row, kept) && all > 0.0; // else no running mass is a number
         double mass = all;
-        Candidate end{};
+        Candidate end{}, drawn{};
         bool known = false; // `end` is the last kept candidate
-        if (kept < n) {
-            end = find(Place{kRank, (uint32_t) kept - 1u, 0.0});
-            known = true;
-            mass = end.massThrough;
-        }
-        if (sums && a.top_p < 1.f) {
-            const Candidate c = find(Place{kReaches, 0u, (double) a.top_p * mass});
-            if ((int) c.rank < kept - 1 || !known) {
+        bool found = false;
+        // the places one after another, in a loop so that the search is there once
+        enum { kTopK, kTopP, kDraw, kEnd };
+        for (int step = kTopK; step <= kEnd; ++step) {
+            const bool wanted = step == kTopK   ? kept < n
+                                : step == kTopP ? sums && a.top_p < 1.f
+                                : step == kDraw ? sums
+                                                : !found && !known;
+            if (!wanted)
+                continue;
+            const Place place = step == kTopP   ? Place{kReaches, 0u, (double) a.top_p * mass}
+                                : step == kDraw ? Place{kPasses, 0u, uniform * mass}
+                                                : Place{kRank, (uint32_t) kept - 1u, 0.0};
+            // its bin, and the candidate among the bin's gathered ones.  The
+            // bins' running masses and `mass` are different sums of the same
+            // weights: the largest draws may lie past the last kept
+            // candidate's bin, where nothing is kept (or gathered)
+            const Span span = find_bin(bins, place, 0u, 0.0);
+            if (step == kDraw && (int) span.before >= kept)
+                continue;
+            const Candidate c = locate(w.gathered + span.before, span, place, inverse, top, bins, ranks);
+            if (span.count > (uint32_t) kRankCap) // `locate` has used the bins' space
+                load_bins(w, bins);
+            if (step == kDraw) {
+                drawn = c;
+                found = (int) c.rank < kept;
+            } else if (step != kTopP || (int) c.rank < kept - 1 || !known) {
                 end = c;
                 known = true;
                 kept = (int) c.rank + 1;
                 mass = c.massThrough;
             }
         }
-        bool drawn = false;
-        if (sums) {
-            // the bins' running masses and `mass` are different sums of the same
-            // weights: the largest draws may lie past the last kept candidate's
-            // bin, where nothing is kept (or gathered)
-            const Place place{kPasses, 0u, uniform * mass};
-            const Span span = find_bin(bins, place, 0u, 0.0);
-            if ((int) span.before < kept) {
-                const Candidate c = find_in(span, place);
-                drawn = (int) c.rank < kept;
-                chosen = c.token;
-            }
-        }
-        if (!drawn) {
-            if (!known)
-                end = find(Place{kRank, (uint32_t) kept - 1u, 0.0});
-            chosen = end.token;
-        }
+        chosen = found ? drawn.token : end.token;
     }
     if (t == 0) {
         if (a.sequence)
@@ -943,7 +941,7 @@ SampleWorkspace carve(void *workspace, int vocab)
         p += align256(bytes);
         return at;
     };
-    w.row = reinterpret_cast<ChunkState *>(take(sizeof(ChunkState)));
+    w.row = reinterpret_cast<RowState *>(take(sizeof(RowState)));
     w.summary = reinterpret_cast<Gathered *>(take(sizeof(Gathered)));
     w.chunks = reinterpret_cast<ChunkState *>(take(w.chunkCount * sizeof(ChunkState)));
     w.counts = reinterpret_cast<uint32_t *>(take(kBins * sizeof(uint32_t)));
@@ -960,7 +958,7 @@ size_t sample_workspace_bytes(int vocab)
 {
     if (vocab <= 0)
         return 0;
-    return align256(sizeof(ChunkState)) + align256(sizeof(Gathered)) + align256(sample_chunks(vocab) * sizeof(ChunkState))
+    return align256(sizeof(RowState)) + align256(sizeof(Gathered)) + align256(sample_chunks(vocab) * sizeof(ChunkState))
            + 2 * align256(kBins * sizeof(uint32_t)) + 2 * align256(kBins * sizeof(uint64_t))
            + align256((size_t) vocab * sizeof(uint64_t)) + 256; // and its alignment
 }

@@ -798,7 +798,11 @@ __global__ __launch_bounds__(kThreads) void mqa_partial_kernel(
 // splits three times through memory, took 57 us for a row of 8000 keys.)  Few
 // rows take one-wave workgroups of 64 channels, so a row's partials come over
 // many compute units (63 splits of one row: 9.5 -> 5.2 us); many rows 512
-// channels a workgroup, which start fewer and share the factors.
+// channels a workgroup, which start fewer and share the factors.  Heads of
+// less than 64 channels share a wave there, one after another: rows of up to
+// some 100 keys end 0.5 to 3 us later than in one workgroup of 256 threads a
+// row, rows of 2000 keys 15 to 20 us sooner (8 heads of 32: 8.0 -> 9.2, 28 ->
+// 12.5); 256 and 1024 threads for those lose 2 to 7 us of the latter.
 // tiled: the rows' splits are launch_tiled_attention's (rows it finished
 // itself are left alone), else mqa_partial_kernel's.
 template <int T, int C>

@@ -915,8 +915,9 @@ __global__ __launch_bounds__(kThreads) void geglu_kernel(const float *__restrict
 // Eight outputs a thread (geglu_kernel's values and bytes): the one-output form
 // computes each block's scale 32 times over and stores a byte a lane.  Threads
 // run over the pieces of all rows, so a width that is no multiple of a
-// workgroup's leaves none of them idle.  2048 rows of 16384: 144 -> 88 us (304
-// MB, which the copy rate allows in 62).
+// workgroup's leaves none of them idle (16384 rows of 512 32.8 -> 23.3 us, a
+// grid of rows 27.5; 32768 rows of 32 16.9 -> 5.6, a grid of rows 47).  2048 rows of
+// 16384: 144 -> 89 us (304 MB, which the copy rate allows in 62).
 __global__ __launch_bounds__(kThreads) void geglu_wide_kernel(const float *__restrict__ fused,
                                                               int rows, int intermediate,
                                                               float *__restrict__ out,

@@ -11,10 +11,10 @@
 //
 // Nothing sorts the row.  Each step needs one place in the ranking (the k-th
 // candidate, the one that reaches a mass), so the row is spread over 2048
-// bins (BinRule) whose order is the ranking's; a
-// scan of the bins' counts and masses gives the bin that holds the place, and
-// that bin's candidates alone are ranked.  The bins' width follows the row's
-// spread, so a flat row or one of equal logits fills them too.  A bin past
+// bins (BinRule) whose order is the ranking's; a scan of the bins' counts and
+// masses gives the bin that holds the place, and that bin's candidates alone
+// are ranked.  The bins' width follows the row's spread, so a flat row or one
+// of equal logits fills them too.  A bin past
 // kRankCap candidates (a crowd of near ties below an outlier) is spread over
 // 2048 bins again, of the range its (score, token) keys cover, until few
 // enough are left: some passes of one workgroup over its candidates.  Four
@@ -35,12 +35,13 @@
 //
 // The launches are bound by their chains (a read of the chunk's 16 KB, the
 // atomics, the scans), not by the row's 1 MB.  A row of 256 000 normal logits
-// (sigma 3) at temperature 0.8, top-k 40, top-p 0.95: 46 us (4, 13, 12
-// and 5 in the kernels); the eight-pass radix sort of the row, its
-// one-workgroup scans and the draw over the ranked row had taken 811.  256 000
-// equal logits with these options: 56 us (the sort 724; with bins of one width
-// for all rows, all candidates in one of them, 2300).  255 999 logits within
-// 1e-5 of each other below an outlier, top-k 1000: 715 (the sort 728).
+// (sigma 3) at temperature 0.8, top-k 40, top-p 0.95: 46.6 us (4, 14, 12
+// and 5 in the kernels; 1 of them for the row's spread); an eight-pass radix
+// sort of the row, its one-workgroup scans and the draw over the ranked row
+// had taken 811.  256 000 equal logits at temperature 1: 56 us (the sort 724;
+// with bins of one width for all rows, all candidates in one of them, 2300).
+// 255 999 logits within 1e-5 of each other below an outlier, temperature 4,
+// top-k 1000: 717 (the sort 728).
 #include "gq8_device.hpp"
 #include "gq8_kernels.hpp"
 #include "gq8_numerics.hpp"

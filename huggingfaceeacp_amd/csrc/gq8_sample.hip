@@ -14,11 +14,10 @@
 // bins (BinRule) whose order is the ranking's; a scan of the bins' counts and
 // masses gives the bin that holds the place, and that bin's candidates alone
 // are ranked.  The bins' width follows the row's spread, so a flat row or one
-// of equal logits fills them too.  A bin past
-// kRankCap candidates (a crowd of near ties below an outlier) is spread over
-// 2048 bins again, of the range its (score, token) keys cover, until few
-// enough are left: some passes of one workgroup over its candidates.  Four
-// launches:
+// of equal logits fills them too.  A bin past kRankCap candidates (a crowd of
+// near ties below an outlier) is spread over 2048 bins again, of the range its
+// (score, token) keys cover, until few enough are left: some passes of one
+// workgroup over its candidates.  Four launches:
 //   sample_max_kernel      each chunk's largest score, unmasked count and last
 //                          unmasked token; the bins cleared
 //   sample_bins_kernel     the chunks' masses; the bins' counts and masses
